@@ -1,6 +1,8 @@
 // Gated GQA attention over a per-sequence KV cache for the 1 + k verify block
 // (gfx950, bf16 MFMA).
 //
+// (Long calls, whose query rows alone fill the chip, go to attn_prefill.hip.)
+//
 // Math (src/qwen3_5/blocks.py:226-235 + src/attention.py:43-51): query i of the T
 // new positions of sequence b sits at absolute position L_b - T + i and attends the
 // keys at positions <= that (offset-causal; plain causal when T == L_b); scores are
@@ -36,34 +38,13 @@
 //     maximum exceeds it by more than 16 in the exponent.
 // At the end of a pair the four waves' (m, l, O) are merged through the free LDS set
 // into the workgroup's piece.
-#include "common.h"
+#include "attn_common.h"
 
 namespace lollm {
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-
-constexpr int AT_D = 256;            // head dim
-constexpr int AT_ROWS = 32;          // MFMA rows per pair (n_rep x QB)
 constexpr int AT_BLOCK = 128;        // keys per block
 constexpr int AT_MAXB = 512;         // sequences per call (prefix table in LDS)
 constexpr int AT_PART = 2 * AT_ROWS + AT_ROWS * AT_D;  // floats per partial
-
-struct AttnArgs {
-  const uint16_t* q;       // (B, T, Hq, D)
-  const uint16_t* kc;      // K cache
-  const uint16_t* vc;      // V cache
-  const int32_t* kv_len;   // (B) keys per sequence, the T new ones included
-  const uint16_t* gate;    // (B, T, Hq * D) or null
-  uint16_t* out;           // (B, T, Hq * D)
-  float* ws;               // partials: (nw + pairs) x AT_PART, then the combine table
-  long long seq_stride, head_stride;  // cache strides in elements
-  int B, T, Hq, Hkv, n_rep, QB, qblocks, max_len, nw;
-  float cl2;               // scale * log2(e)
-};
-
-__device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
-
-__device__ __forceinline__ float sigmoidf_(float x) { return 1.f / (1.f + __expf(-x)); }
 
 __device__ __forceinline__ int seq_len(const AttnArgs& a, int b) {
   return min(max(a.kv_len[b], 0), a.max_len);  // never past the cache capacity
@@ -102,12 +83,6 @@ constexpr int AW_VSET = AW_WAVES * AW_VWAVE;          // the V rows of one block
 constexpr int AW_QROW = AT_D * 2 + 16;                // padded Q row in LDS
 constexpr int AW_OROW = AT_D / 2 + 4;                 // padded floats per row of an O half-dump
 static_assert(AW_WAVES * AT_ROWS * AW_OROW * 4 <= AW_VSET, "the O dump fits a V set");
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-typedef unsigned int u32x2_t __attribute__((ext_vector_type(2)));
-typedef __attribute__((address_space(3))) void lds_void_t;
-typedef __attribute__((address_space(3))) s16x4 lds_s16x4_t;
 
 // pre[b] = blocks of sequences 0..b-1 (pre[0] = 0), for b = 0..B, and len[b] = the
 // clamped key count of sequence b, built in LDS by the whole workgroup (so the main
@@ -595,6 +570,10 @@ LOLLM_API int lollm_attn_verify(const void* q, const void* k_cache, const void* 
   a.max_len = max_len; a.nw = nw;
   a.cl2 = scale * 1.4426950408889634f;
   hipStream_t st = (hipStream_t)stream;
+  if (grid == 0) {
+    const int groups = attn_prefill_groups(B, T, Hkv, n_rep, max_len, nw);
+    if (groups) return attn_prefill_launch(a, groups, st);
+  }
   hipLaunchKernelGGL(attn_verify_kernel, dim3(nw), dim3(AW_THREADS), 0, st, a);
   if ((rc = launch_status())) return rc;
   hipLaunchKernelGGL(attn_combine_kernel, dim3(AT_ROWS, B * Hkv * qblocks), dim3(256), 0, st, a);

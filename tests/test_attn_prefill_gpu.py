@@ -1,0 +1,100 @@
+"""The long-call attention kernel (many new positions per sequence) and the many-token
+attention prologue, against the oracle and against the kernels of the short calls.
+
+An explicit `grid` always takes the split-K kernels, so the same operands reach both."""
+
+import pytest
+import torch
+
+from test_attn_gpu import D, TOL, make_case, oracle
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # B, T, Hq, Hkv, lens
+    (2, 16, 8, 2, [16, 40]),            # the shortest long call; 64 rows of a 128-row tile
+    (1, 17, 32, 4, [17]),               # one row past a tile (16 positions x 8 heads)
+    (2, 33, 4, 4, [33, 500]),           # n_rep 1: 33 rows
+    (1, 43, 6, 2, [75]),                # n_rep 3: 42 positions per tile, 2 rows of it unused
+    (1, 50, 32, 1, [64]),               # n_rep 32: 4 positions per tile
+    (3, 100, 10, 2, [100, 131, 160]),   # n_rep 5; key blocks cut at every residue
+    (1, 31, 8, 2, [511]),               # one position short of a block end
+    (2, 64, 8, 2, [64, 20]),            # kv_len < T: the first rows see no key
+    (2, 16, 8, 2, [16, 0]),             # an empty sequence
+    (1, 2053, 8, 2, [2053]),            # many tiles, odd sizes
+    (4, 200, 32, 4, [200, 900, 333, 1200]),
+]
+
+
+@pytest.mark.parametrize("B,T,Hq,Hkv,lens", CASES)
+@pytest.mark.parametrize("gated", [True, False])
+def test_long_call_matches_oracle_and_split(B, T, Hq, Hkv, lens, gated):
+    from lollm_amd import ops
+    print(f"case long attention B={B} T={T} Hq={Hq} Hkv={Hkv} lens={lens} gated={gated}", flush=True)
+    q, kc, vc, kl, gate = make_case(B, T, Hq, Hkv, lens, seed=sum(lens) + T, max_len=max(lens) + 3)
+    gd = gate.cuda() if gated else None
+    out = ops.attn_verify(q.cuda(), kc.cuda(), vc.cuda(), kl.cuda(), gd)
+    split = ops.attn_verify(q.cuda(), kc.cuda(), vc.cuda(), kl.cuda(), gd, grid=64)
+    torch.cuda.synchronize()
+    assert torch.isfinite(out.float()).all()
+    # both round P to bf16 against their own running maxima and the result once: two bf16
+    # roundings of P (relative 2^-9) and one of the output
+    torch.testing.assert_close(out.float(), split.float(), rtol=1.6e-2, atol=1e-2)
+    if all(L >= T for L in lens):
+        torch.testing.assert_close(out.cpu().float(), oracle(q, kc, vc, kl, gate if gated else None), **TOL)
+
+
+def test_two_row_groups_match_oracle():
+    """Enough 256-row tiles for the 64-rows-per-wave form (448 of them on 256 CUs), odd
+    lengths; two of the sequences against the oracle, all against the split kernels."""
+    from lollm_amd import ops
+    B, T, Hq, Hkv = 16, 231, 32, 4
+    lens = [T + 37 * b for b in range(B)]
+    print("case two row groups", flush=True)
+    q, kc, vc, kl, gate = make_case(B, T, Hq, Hkv, lens, seed=5, max_len=max(lens) + 1)
+    out = ops.attn_verify(q.cuda(), kc.cuda(), vc.cuda(), kl.cuda(), gate.cuda())
+    split = ops.attn_verify(q.cuda(), kc.cuda(), vc.cuda(), kl.cuda(), gate.cuda(), grid=256)
+    torch.testing.assert_close(out.float(), split.float(), rtol=1.6e-2, atol=1e-2)
+    pick = [0, 15]
+    torch.testing.assert_close(out[pick].cpu().float(),
+                               oracle(q[pick], kc[pick], vc[pick], kl[pick], gate[pick]), **TOL)
+
+
+def test_large_scores_move_the_reference_maximum():
+    """Keys whose scores grow along the context: the running maximum moves often, by far more
+    than the rescale threshold, and differently per row."""
+    from lollm_amd import ops
+    B, T, Hq, Hkv = 1, 300, 8, 2
+    q, kc, vc, kl, gate = make_case(B, T, Hq, Hkv, [300], seed=9)
+    kc = (kc.float() * torch.linspace(0.2, 12, 300)[None, None, :, None]).bfloat16()
+    print("case growing scores", flush=True)
+    out = ops.attn_verify(q.cuda(), kc.cuda(), vc.cuda(), kl.cuda(), gate.cuda())
+    torch.testing.assert_close(out.cpu().float(), oracle(q, kc, vc, kl, gate), **TOL)
+
+
+@pytest.mark.parametrize("B,T,Hq,Hkv,rd,rope", [(2, 150, 8, 2, 64, None), (4, 64, 5, 2, 256, "start"),
+                                               (3, 100, 4, 1, 16, "token"), (2, 128, 3, 3, 0, None),
+                                               (2, 130, 4, 2, 128, "token")])
+def test_many_token_prologue_equals_few_token_prologue(B, T, Hq, Hkv, rd, rope):
+    """256 tokens or more take the token-per-workgroup kernel; the same tokens in calls of
+    fewer take the head-per-workgroup kernel.  Same bits, also at the cache's end."""
+    from lollm_amd import ops
+    print(f"case prologue B={B} T={T} Hq={Hq} Hkv={Hkv} rd={rd} rope={rope}", flush=True)
+    g = torch.Generator().manual_seed(B * T)
+    max_len = T + 20
+    qkv = torch.randn(B, T, Hq * 2 * D + 2 * Hkv * D, generator=g).bfloat16().cuda()
+    qn, kn = ((0.1 * torch.randn(D, generator=g)).bfloat16().cuda() for _ in range(2))
+    freq = (1.0 / (1e7 ** (torch.arange(0, max(rd, 2), 2).float() / max(rd, 2)))).cuda()
+    lengths = torch.randint(0, 30, (B,), generator=g, dtype=torch.int32).cuda()   # some rows past max_len
+    pos = {None: None, "start": torch.randint(0, 40000, (B,), generator=g, dtype=torch.int32),
+           "token": torch.randint(0, 40000, (B, T), generator=g, dtype=torch.int32)}[rope]
+    kc, vc = (torch.zeros(B, Hkv, max_len, D, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    kc2, vc2 = torch.zeros_like(kc), torch.zeros_like(vc)
+    q, gate = ops.attn_prologue(qkv, qn, kn, freq, lengths, B, T, Hq, Hkv, D, rd, 1e-6, kc, vc,
+                                rope_pos=None if pos is None else pos.cuda())
+    for b in range(B):
+        q1, g1 = ops.attn_prologue(qkv[b:b + 1].contiguous(), qn, kn, freq, lengths[b:b + 1].clone(), 1, T, Hq,
+                                   Hkv, D, rd, 1e-6, kc2[b:b + 1], vc2[b:b + 1],
+                                   rope_pos=None if pos is None else pos[b:b + 1].cuda())
+        assert torch.equal(q1[0].cpu(), q[b].cpu()) and torch.equal(g1[0].cpu(), gate[b].cpu())
+    assert torch.equal(kc.cpu(), kc2.cpu()) and torch.equal(vc.cpu(), vc2.cpu())

@@ -359,6 +359,21 @@ int lollm_gdn_layer_chunked(const void* proj, long long proj_stride, const void*
                             int fresh, void* out, int B, int T, int Hk, int Hv, int Dk, int Dv,
                             int conv_kernel, float eps, void* stream);
 
+/* lollm_gdn_layer_chunked with the chunks of a head spread over the chip: the part of every
+ * chunk that does not depend on the state is formed for all chunks at once, and a short
+ * recurrence over the chunks follows (calls with few (sequence, head) pairs, which otherwise
+ * leave most CUs idle).  Same arguments, support and results up to summation order.
+ *   workspace  lollm_gdn_split_workspace_bytes() bytes, 16-byte aligned (required); used
+ *              only within the call.  -1: bad sizes */
+long long lollm_gdn_split_workspace_bytes(int B, int T, int Hk, int Hv);
+int lollm_gdn_layer_split(const void* proj, long long proj_stride, const void* conv_w,
+                          const float* A_log, const float* dt_bias, const void* norm_w,
+                          void* win, const int32_t* conv_off, int win_rows, float* rec,
+                          const int32_t* rec_half, void* rep, const int32_t* replay, int slots,
+                          int fresh, void* out, void* workspace, long long workspace_bytes, int B,
+                          int T, int Hk, int Hv, int Dk, int Dv, int conv_kernel, float eps,
+                          void* stream);
+
 /* Greedy acceptance (temperature 0) without the verify logits: argmax (B, k + 1) int32
  * holds the argmax token of each verify row (lollm_gemm_argmax on the lm_head, same
  * token as lollm_gemm + the greedy sampler); n_accepted[b] = the number of leading drafts

@@ -59,6 +59,10 @@ SIGNATURES = {
                          _I, _P, _I, _I, _I, _I, _I, _I, _I, _F, _P], _I),
     "lollm_gdn_layer_chunked": ([_P, ctypes.c_longlong, _P, _P, _P, _P, _P, _P, _I, _P, _P, _P,
                                  _P, _I, _I, _P, _I, _I, _I, _I, _I, _I, _I, _F, _P], _I),
+    "lollm_gdn_split_workspace_bytes": ([_I, _I, _I, _I], ctypes.c_longlong),
+    "lollm_gdn_layer_split": ([_P, ctypes.c_longlong, _P, _P, _P, _P, _P, _P, _I, _P, _P, _P,
+                               _P, _I, _I, _P, _P, ctypes.c_longlong, _I, _I, _I, _I, _I, _I, _I,
+                               _F, _P], _I),
     "lollm_gdn_state": ([_P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _P], _I),
     "lollm_gemm_tile_weights": ([_P, _P, _I, _I, _I, _P], _I),
     "lollm_gemm_workspace_bytes": ([_I, _I, _I, _I], ctypes.c_longlong),

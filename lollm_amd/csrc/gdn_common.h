@@ -101,6 +101,13 @@ __device__ __forceinline__ uint4 gdn_record_kv(const float* act_row_k, int part)
 // long-call kernels start from (defined in gdn_layer.hip).
 int gdn_long_call_prologue(const GdnLayerArgs& a, int B, hipStream_t stream);
 
+// The checks and the argument block of a chunked long call (defined in gdn_chunk.hip).
+int gdn_long_call_args(GdnLayerArgs& a, const void* proj, long long proj_stride, const void* conv_w,
+                       const float* A_log, const float* dt_bias, const void* norm_w, void* win,
+                       const int32_t* conv_off, int win_rows, float* rec, const int32_t* rec_half, void* rep,
+                       const int32_t* replay, int slots, int fresh, void* out, int B, int T, int Hk, int Hv,
+                       int Dk, int Dv, int conv_kernel, float eps);
+
 // SiLU with the hardware reciprocal: within 1.5 ulp (fp32) of x / (1 + e^-x), below the
 // resolution of the bf16 values it feeds
 __device__ __forceinline__ float silu_g(float x) { return x * __builtin_amdgcn_rcpf(1.f + __expf(-x)); }

@@ -606,7 +606,13 @@ def attn_small(qkv, q_norm_w, k_norm_w, inv_freq, lengths, kv_len, B, Hq, Hkv, D
     return out
 
 
-GDN_CHUNK_MIN_T = 64
+# Long calls that take the chunked form: a chunk costs a workgroup about the same time whatever
+# it holds, the recurrence 2.2 us per token and round of heads (us, chunked / recurrent, 32
+# heads a sequence: 24 tokens x 1 sequence 27 / 58, x 64 255 / 316; 12 tokens x 8 34 / 45, x 32
+# 127 / 106; 63 tokens x 1 28 / 141).
+GDN_CHUNK_MIN_T = 24
+GDN_CHUNK_MIN_T_FEW = 12
+GDN_CHUNK_FEW_HEADS = 256
 
 
 def gdn_chunked_ok(T, slots, win_rows, conv_kernel, proj_stride=0):
@@ -615,6 +621,14 @@ def gdn_chunked_ok(T, slots, win_rows, conv_kernel, proj_stride=0):
     projection rows addressable with 32-bit byte offsets."""
     return (conv_kernel == 4 and T > slots and conv_kernel - 1 + T > win_rows
             and T * proj_stride * 2 < 2 ** 31)
+
+
+# Heads of a call (B * Hv) up to which its chunks, when there are several, are spread over the
+# chip; more heads fill it walking their own chunks (us, spread / walked, 32 heads a sequence:
+# 1 x 1847 tokens 146 / 543, 3 x 1500 274 / 453, 4 x 1000 229 / 308, 5 x 1638 515 / 499,
+# 8 x 1024 461 / 320; 1 x 100 32 / 46, 1 x 64 28 / 28).
+GDN_SPLIT_MAX_HEADS = 128
+GDN_CHUNK = 64
 
 
 def gdn_record_bytes(D):
@@ -639,8 +653,9 @@ def gdn_layer(proj, conv_w, A_log, dt_bias, norm_w, win, conv_off, rec, rec_half
     """Fused GDN mixer (include/lollm_amd.h).  proj (B, T, P) bf16; win (B, 2W,
     conv_dim) bf16; rec (B, 2, Hv, D, D) fp32 state halves; rep (B, 2, Hv, S,
     gdn_record_bytes(D)) uint8 replay records; conv_off / rec_half / replay (B,) int32.
-    chunked: None = the chunked kernel for long calls of at least GDN_CHUNK_MIN_T tokens
-    that it supports, the recurrent kernel otherwise; True / False force one."""
+    chunked: None = the chunked kernels for long calls of at least GDN_CHUNK_MIN_T tokens
+    (GDN_CHUNK_MIN_T_FEW with few heads) that they support, the recurrent kernel otherwise;
+    True / False force one."""
     P = proj.shape[-1]
     _need(proj, "proj", torch.bfloat16)
     _need(win, "win", torch.bfloat16)
@@ -653,12 +668,18 @@ def gdn_layer(proj, conv_w, A_log, dt_bias, norm_w, win, conv_off, rec, rec_half
         out = torch.empty(B, T, value_dim, dtype=torch.bfloat16, device=proj.device)
     W = win.shape[1] // 2
     if chunked is None:
-        chunked = T >= GDN_CHUNK_MIN_T and gdn_chunked_ok(T, S, W, conv_kernel, P)
-    fn = "lollm_gdn_layer_chunked" if chunked else "lollm_gdn_layer"
+        chunked = (T >= (GDN_CHUNK_MIN_T_FEW if B * Hv <= GDN_CHUNK_FEW_HEADS else GDN_CHUNK_MIN_T)
+                   and gdn_chunked_ok(T, S, W, conv_kernel, P))
+    fn, ws = "lollm_gdn_layer_chunked" if chunked else "lollm_gdn_layer", ()
+    if chunked and T > GDN_CHUNK and B * Hv <= GDN_SPLIT_MAX_HEADS:
+        need = _lib.lib().lollm_gdn_split_workspace_bytes(B, T, Hk, Hv)
+        if need > 0:
+            buf = torch.empty(need, dtype=torch.uint8, device=proj.device)
+            fn, ws = "lollm_gdn_layer_split", (_ptr(buf), need)
     rc = getattr(_lib.lib(), fn)(
         _ptr(proj), P, _ptr(conv_w), _ptr(A_log), _ptr(dt_bias), _ptr(norm_w), _ptr(win),
         _ptr(conv_off), W, _ptr(rec), _ptr(rec_half), _ptr(rep), _ptr(replay), S,
-        int(bool(fresh)), _ptr(out), B, T, Hk, Hv, D, D, conv_kernel, float(eps), _stream())
+        int(bool(fresh)), _ptr(out), *ws, B, T, Hk, Hv, D, D, conv_kernel, float(eps), _stream())
     _lib.check(rc, fn)
     return out
 

@@ -374,6 +374,14 @@ int lollm_gdn_layer_split(const void* proj, long long proj_stride, const void* c
                           int T, int Hk, int Hv, int Dk, int Dv, int conv_kernel, float eps,
                           void* stream);
 
+/* C = A W^T (bf16, fp32 sums) for many rows, W from lollm_gemm_tile_weights with the same
+ * epilogue: 0 C is (M, N); 1 W = [gate; up], C is (M, N / 2) = silu(gate) * up with
+ * lollm_gemm's rounding points.  tile: the output tile of a workgroup as 10 x rows / 64 +
+ * columns / 64, one of 44, 34, 43, 24 (it changes the time only).  N a multiple of 64, K of
+ * 128, lda and ldc of 8; A, Wt and C 16-byte aligned. */
+int lollm_gemm_rows(const void* A, long long lda, const void* Wt, void* C, long long ldc, int M,
+                    int N, int K, int epilogue, int tile, void* stream);
+
 /* Greedy acceptance (temperature 0) without the verify logits: argmax (B, k + 1) int32
  * holds the argmax token of each verify row (lollm_gemm_argmax on the lm_head, same
  * token as lollm_gemm + the greedy sampler); n_accepted[b] = the number of leading drafts

@@ -8,6 +8,8 @@ and launches on `torch.cuda.current_stream()`.
 
 from __future__ import annotations
 
+import functools
+
 import torch
 
 from . import _lib
@@ -248,6 +250,55 @@ def gemm(x, tiled, N, K, epilogue=GEMM_NONE, out=None, grid=0):
     rc = _lib.lib().lollm_gemm(_ptr(x), K, _ptr(tiled), _ptr(out), oc, M, N, K, epilogue, _ptr(ws),
                                ws.numel(), grid, _stream())
     _lib.check(rc, "lollm_gemm")
+    return out
+
+
+# lollm_gemm_rows: us per k32 step of a tile with every CU busy (3998 rows, random values), and
+# the steps an epilogue costs
+GEMM_ROWS_STEP_US = {44: 0.66, 34: 0.52, 43: 0.52, 24: 0.37}
+GEMM_ROWS_EPILOGUE_STEPS = 10
+
+
+@functools.lru_cache(maxsize=4096)
+def gemm_rows_tile(M, N, K, epilogue, cus):
+    """The lollm_gemm_rows tile for this product on a device with `cus` CUs, or 0 where the
+    library's is the faster one.  The tile with the least estimated time: whole rounds of the
+    chip at the step times above, a last round in part at 0.72 of one plus its share (a chip
+    that is not full runs each step faster).
+    Too few tiles leave CUs idle, where the library splits K: from 0.6 of the CUs on this
+    kernel is as fast (N = 4096, rows: 1024 0.77 of the library's speed, 1536 0.94 - 1.04, 1847
+    1.05 - 1.12).  One full round of 256 x 256 tiles is the library's best case (N = 4096, 3998
+    rows: 0.97); everywhere else its rounds are less even (4500 rows 1.0 - 1.9, N = 12352 1.0 -
+    1.65, N = 18432 0.98 - 1.36)."""
+    best, tile, count = None, 0, 0
+    for t, us in GEMM_ROWS_STEP_US.items():
+        n = -(-M // (64 * (t // 10))) * -(-N // (64 * (t % 10)))
+        part = (n % cus) / cus
+        cost = (n // cus + (0.72 + 0.28 * part if part else 0.0)) * (K // 32 + GEMM_ROWS_EPILOGUE_STEPS) * us
+        if best is None or cost < best:
+            best, tile, count = cost, t, n
+    if 10 * count < 6 * cus:
+        return 0
+    whole = -(-M // 256) * -(-N // 256)
+    if epilogue == GEMM_NONE and 100 * whole >= 93 * cus and whole <= cus:
+        return 0
+    return tile
+
+
+def gemm_rows(x, tiled, N, K, epilogue, tile):
+    """y = x W^T for many rows x (..., K) bf16; `tiled` from gemm_tile_weights with the same
+    epilogue (GEMM_SWIGLU: silu(gate) * up), tile from gemm_rows_tile."""
+    M = x.numel() // K
+    if x.shape[-1] != K:
+        raise ValueError(f"x has {x.shape[-1]} features, expected {K}")
+    x = x.contiguous()
+    _need(x, "x", torch.bfloat16)
+    _need(tiled, "tiled", torch.bfloat16, (N * K,))
+    oc = N // 2 if epilogue == GEMM_SWIGLU else N
+    out = torch.empty(*x.shape[:-1], oc, dtype=torch.bfloat16, device=x.device)
+    rc = _lib.lib().lollm_gemm_rows(_ptr(x), K, _ptr(tiled), _ptr(out), oc, M, N, K, epilogue, tile,
+                                    _stream())
+    _lib.check(rc, "lollm_gemm_rows")
     return out
 
 

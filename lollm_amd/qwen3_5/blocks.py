@@ -6,7 +6,8 @@ input are concatenated into one GEMM weight (GDN in_proj_qkv|z|b|a, attention
 q|k|v, MLP gate|up), so a layer issues 4 GEMMs plus fused HIP kernels for everything
 between them.  A GEMM over at most 64 rows (the verify and draft passes) streams a
 tiled copy of its weight through lollm_gemm, with SiLU(gate) * up fused into the
-gate|up GEMM; longer calls (the prefill) use hipBLASLt on the row-major weight.
+gate|up GEMM; longer calls (the prefill) take lollm_gemm_rows on the same copy, SwiGLU
+fused too, where its tiles fill the chip, else hipBLASLt on the row-major weight.
 """
 
 from __future__ import annotations
@@ -24,7 +25,8 @@ def _cat_rows(*ws):
 
 # Fixed GEMM path and grid per projection shape, so a given (weights, inputs) gives the
 # same bits in every process (a timing-based choice could differ between runs and
-# change rounding).  Rows <= 64 take lollm_gemm, rows > 64 (the prefill) hipBLASLt.
+# change rounding).  Rows <= 64 take lollm_gemm, rows > 64 (the prefill) lollm_gemm_rows or
+# hipBLASLt (ops.gemm_rows_tile).
 # lollm_gemm deals 64-column groups x 128-k stages out to one workgroup per CU; when the
 # groups number between 3/4 of the CUs and the CUs, one workgroup per group instead
 # leaves no group cut between workgroups, so no merge launch follows (the GDN in_proj
@@ -36,8 +38,8 @@ def _cat_rows(*ws):
 
 
 def gemm_path(N, K, epilogue, rows, tiled=True):
-    """'gemm' (lollm_gemm) or 'blas' (hipBLASLt) for a projection call; a pure function
-    of the shape."""
+    """'gemm' (lollm_gemm) or 'blas' (lollm_gemm_rows or hipBLASLt) for a projection call; a
+    pure function of the shape."""
     return "gemm" if tiled and rows <= ops.GEMM_MAX_ROWS else "blas"
 
 
@@ -60,7 +62,8 @@ def gemm_grid(N, cus, rows=ops.GEMM_MAX_ROWS):
 
 class Projection:
     """y = x W^T (blocks.py's nn.Linear layers, no bias).  Keeps the row-major weight
-    for hipBLASLt (F.linear) and a tiled copy for lollm_gemm (<= 64 rows).
+    for hipBLASLt (F.linear) and a tiled copy for lollm_gemm (<= 64 rows) and
+    lollm_gemm_rows (more).
     epilogue=GEMM_SWIGLU: W = [gate; up], y = silu(x gate^T) * x up^T (blocks.py:341-342).
     The path of each call is gemm_path() of its shape, the grid gemm_grid()."""
 
@@ -84,6 +87,14 @@ class Projection:
     def path(self, rows):
         return gemm_path(self.N, self.K, self.epilogue, rows, self.tiled is not None)
 
+    def rows_tile(self, x, rows):
+        """The lollm_gemm_rows tile of a call past the few-row GEMM, 0 for hipBLASLt: a pure
+        function of the shape (and 0 where only F.linear serves: another dtype, a gradient)."""
+        if (self.tiled is None or x.dtype != torch.bfloat16 or not x.is_cuda
+                or x.data_ptr() % 16 or (x.requires_grad and torch.is_grad_enabled())):
+            return 0
+        return ops.gemm_rows_tile(rows, self.N, self.K, self.epilogue, _cus())
+
     def argmax_grid(self, rows):
         """Workgroups of the fused lm_head argmax (lollm_gemm_argmax): one per CU."""
         return _cus()
@@ -95,6 +106,9 @@ class Projection:
     def __call__(self, x):
         rows = x.numel() // self.K
         if self.path(rows) == "blas":
+            tile = self.rows_tile(x, rows)
+            if tile:
+                return ops.gemm_rows(x, self.tiled, self.N, self.K, self.epilogue, tile)
             return self._blas(x)
         return ops.gemm(x, self.tiled, self.N, self.K, self.epilogue, grid=self.grid(rows))
 

@@ -1,0 +1,108 @@
+"""The many-row GEMM (lollm_gemm_rows) against fp32, at the edges of its tiles, and its row
+independence of M and tile; the rule that picks its tile is checked on the CPU."""
+
+import pytest
+import torch
+
+TILES = (44, 34, 43, 24)
+
+
+def case(M, N, K, seed):
+    g = torch.Generator().manual_seed(seed)
+    return torch.randn(M, K, generator=g).bfloat16(), (torch.randn(N, K, generator=g) * K ** -0.5).bfloat16()
+
+
+def close(got, ref):
+    # fp32 sums of exact bf16 products, one rounding to bf16 (2^-9 of the value)
+    torch.testing.assert_close(got.float().cpu(), ref, rtol=2 ** -8, atol=1e-3)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("M,N,K", [(1, 64, 128), (65, 64, 128), (129, 320, 256), (255, 256, 384), (257, 192, 128),
+                                   (300, 832, 512), (193, 1088, 128)])
+def test_gemm_rows_matches_fp32(M, N, K, tile):
+    from lollm_amd import ops
+    print(f"case gemm rows M={M} N={N} K={K} tile={tile}", flush=True)
+    x, W = case(M, N, K, seed=M + N + K)
+    t = ops.gemm_tile_weights(W.cuda())
+    out = torch.full((M + 1, N), 7.0, dtype=torch.bfloat16, device="cuda")
+    from lollm_amd import _lib
+    xd = x.cuda()
+    rc = _lib.lib().lollm_gemm_rows(xd.data_ptr(), K, t.data_ptr(), out.data_ptr(), N, M, N, K, 0, tile,
+                                    torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    close(out[:M], x.float() @ W.float().t())
+    assert (out[M] == 7.0).all()          # nothing written past the last row
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("M,N,K", [(130, 448, 256), (517, 1600, 128), (70, 64, 128)])
+def test_gemm_rows_swiglu_equals_product_then_swiglu(M, N, K, tile):
+    """The fused SwiGLU is the separate kernel's arithmetic: same bits."""
+    from lollm_amd import ops
+    print(f"case gemm rows swiglu M={M} N={N} K={K} tile={tile}", flush=True)
+    x, W = case(M, N, K, seed=M + N)
+    W = (W.float() * 4).bfloat16().cuda()
+    x = x.cuda()
+    got = ops.gemm_rows(x, ops.gemm_tile_weights(W, ops.GEMM_SWIGLU), N, K, ops.GEMM_SWIGLU, tile)
+    ref = ops.swiglu(ops.gemm_rows(x, ops.gemm_tile_weights(W), N, K, ops.GEMM_NONE, tile))
+    assert torch.equal(got, ref)
+
+
+@pytest.mark.gpu
+def test_gemm_rows_several_tiles_per_workgroup_and_row_independence():
+    """More tiles than CUs: a workgroup's next tile is loaded during its last one.  Every tile
+    shape, and a call over a part of the rows, gives a row the same bits."""
+    from lollm_amd import ops
+    M, N, K = 2100, 12352, 128
+    print(f"case gemm rows many tiles M={M} N={N} K={K}", flush=True)
+    x, W = case(M, N, K, seed=3)
+    t, xd = ops.gemm_tile_weights(W.cuda()), x.cuda()
+    outs = [ops.gemm_rows(xd, t, N, K, ops.GEMM_NONE, tile) for tile in TILES]
+    close(outs[0], x.float() @ W.float().t())
+    for o in outs[1:]:
+        assert torch.equal(o, outs[0])
+    part = ops.gemm_rows(xd[700:877].contiguous(), t, N, K, ops.GEMM_NONE, 24)
+    assert torch.equal(part, outs[0][700:877])
+
+
+@pytest.mark.gpu
+def test_projection_takes_the_rows_kernel_and_keeps_gradients():
+    from lollm_amd.qwen3_5.blocks import Projection
+    x, W = case(1200, 8192, 256, seed=4)
+    p = Projection(W.cuda())
+    xd = x.cuda()
+    assert p.rows_tile(xd, 1200) and not p.rows_tile(xd.float(), 1200)
+    close(p(xd), x.float() @ W.float().t())
+    xg = xd.clone().requires_grad_()
+    p(xg).float().sum().backward()
+    assert xg.grad is not None
+
+
+def test_rows_tile_rule():
+    """A pure function of the shape; the library keeps what leaves CUs idle or is one full round
+    of its 256 x 256 tiles."""
+    from lollm_amd import ops
+    assert ops.gemm_rows_tile(128, 4096, 4096, 0, 256) == 0
+    assert ops.gemm_rows_tile(1024, 1024, 3072, 0, 256) == 0
+    assert ops.gemm_rows_tile(3998, 4096, 4096, 0, 256) == 0
+    assert ops.gemm_rows_tile(3998, 4096, 4096, 1, 256) == 44
+    assert ops.gemm_rows_tile(4500, 4096, 12288, 0, 256) == 34
+    assert ops.gemm_rows_tile(2048, 18432, 4096, 0, 256) == 43
+    assert ops.gemm_rows_tile(1847, 4096, 4096, 0, 256) == 24
+    for M in range(65, 9000, 97):
+        for N, K in ((12352, 4096), (18432, 4096), (24576, 4096), (4096, 12288), (1024, 3072)):
+            assert ops.gemm_rows_tile(M, N, K, 0, 256) in (0, *TILES)
+
+
+def test_gemm_rows_refuses_bad_arguments():
+    """Before any HIP call, so without a device."""
+    from lollm_amd import _lib
+    f = _lib.lib().lollm_gemm_rows
+    ok = (16, 128, 16, 16, 64, 1, 64, 128, 0, 44, None)
+    for i, v in ((0, None), (2, None), (3, None), (5, 0), (6, 96), (7, 64), (1, 64), (1, 132), (4, 32), (8, 2), (0, 8)):
+        a = list(ok)
+        a[i] = v
+        assert f(*a) == 1, (i, v)

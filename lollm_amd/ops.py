@@ -30,10 +30,16 @@ def _ptr(t):
 
 
 def _stream():
-    return torch.cuda.current_stream().cuda_stream
+    """The current stream's handle (torch.cuda.current_stream().cuda_stream without building the
+    Stream object: 2 us of the 9 that a call of a small kernel costs the host)."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _need(t: torch.Tensor, name: str, dtype=None, shape=None):
+    # the common case first, without a message or a copied shape
+    if (t.is_cuda and t.is_contiguous() and (dtype is None or t.dtype is dtype)
+            and (shape is None or t.shape == shape) and not t.data_ptr() % 16):
+        return
     if not t.is_cuda:
         raise ValueError(f"{name} must be a HIP device tensor")
     if not t.is_contiguous():
@@ -206,6 +212,12 @@ def gemm_tile_weights(weight, epilogue=GEMM_NONE):
 
 
 def gemm_workspace_bytes(M, N, K, grid=0):
+    return _gemm_workspace_bytes(M, N, K, grid, torch._C._cuda_getDevice() if grid <= 0 else -1)
+
+
+@functools.lru_cache(maxsize=4096)
+def _gemm_workspace_bytes(M, N, K, grid, device):
+    """By sizes, and by device where the grid is its CU count."""
     n = _lib.lib().lollm_gemm_workspace_bytes(M, N, K, grid)
     if n < 0:
         raise ValueError("unsupported GEMM shape")
@@ -219,7 +231,7 @@ def gemm_workspace(nbytes, device):
     """The shared piece buffer of lollm_gemm (one per device, grown on demand; models
     reserve their largest size when they are built).  A buffer that is outgrown is kept
     alive, never freed: a HIP graph captured earlier may still write to its address."""
-    key = torch.device(device)
+    key = device if isinstance(device, torch.device) else torch.device(device)
     ws = _gemm_ws.get(key)
     if ws is None or ws.numel() < nbytes:
         if ws is not None:
@@ -384,7 +396,7 @@ def gemm_rmsnorm_supported(M, N, K, grid=0):
     if not gemm_supported(N, K) or N > 8192 or not 0 < M <= GEMM_MAX_ROWS:
         return False
     if grid <= 0:
-        dev = torch.cuda.current_device()
+        dev = torch._C._cuda_getDevice()
         if dev not in _cu_count:
             _cu_count[dev] = torch.cuda.get_device_properties(dev).multi_processor_count
         grid = 2 * _cu_count[dev]

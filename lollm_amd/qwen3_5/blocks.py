@@ -12,6 +12,8 @@ fused too, where its tiles fill the chip, else hipBLASLt on the row-major weight
 
 from __future__ import annotations
 
+import functools
+
 import torch
 import torch.nn.functional as F
 
@@ -43,6 +45,7 @@ def gemm_path(N, K, epilogue, rows, tiled=True):
     return "gemm" if tiled and rows <= ops.GEMM_MAX_ROWS else "blas"
 
 
+@functools.lru_cache(maxsize=4096)
 def gemm_grid(N, cus, rows=ops.GEMM_MAX_ROWS):
     """Workgroups of a lollm_gemm call with N output columns and `rows` rows on a device
     with `cus` CUs: one per 64-column group when that covers 3/4 of the CUs or more; else
@@ -136,7 +139,7 @@ _CUS = {}
 
 def _cus():
     """Compute units of the current device (the one-workgroup-per-CU GEMM grid)."""
-    dev = torch.cuda.current_device()
+    dev = torch._C._cuda_getDevice()
     if dev not in _CUS:
         _CUS[dev] = torch.cuda.get_device_properties(dev).multi_processor_count
     return _CUS[dev]

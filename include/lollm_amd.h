@@ -432,6 +432,13 @@ int lollm_repetition_penalty(void* logits, long long ld, int B, int T, int V, co
                              int words, const int32_t* extra, int extra_stride, int n_extra0,
                              float penalty, void* stream);
 
+/* y = a copy of one bf16 logit row x (V tokens, V a multiple of 8, both 16-byte aligned) with
+ * the repetition penalty of lollm_repetition_penalty applied to the n tokens of host_tokens
+ * (host memory, read before the call returns; duplicates once, ids outside [0, V) ignored).
+ * n at most 896, else LOLLM_EUNSUPPORTED. */
+int lollm_penalised_row(const void* x, void* y, int V, const int32_t* host_tokens, int n,
+                        float penalty, void* stream);
+
 /* seen[b] |= { tok[b * tok_stride + i] : i < n } for b < B (tokens outside [0, V) ignored):
  * builds the repetition-penalty context of lollm_repetition_penalty from a prompt or a
  * token list.  Replaces: the context list of src/generate.py:45,56 / mtp.py:108,129. */

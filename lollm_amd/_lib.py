@@ -81,6 +81,7 @@ SIGNATURES = {
                            _P, _P, _P, _I, _P], _I),
     "lollm_repetition_penalty": ([_P, ctypes.c_longlong, _I, _I, _I, _P, _I, _P, _I, _I, _F, _P],
                                  _I),
+    "lollm_penalised_row": ([_P, _P, _I, _P, _I, _F, _P], _I),
     "lollm_seen_mark": ([_P, _I, _I, _P, ctypes.c_longlong, _I, _I, _P], _I),
 }
 

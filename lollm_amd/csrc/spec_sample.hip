@@ -50,6 +50,8 @@
 // one-hot (argmax drafts) and 128-bit when q is a sampled distribution.
 #include "common.h"
 
+#include <string.h>
+
 #include <algorithm>
 #include <mutex>
 
@@ -1031,6 +1033,41 @@ __global__ __launch_bounds__(256) void repetition_penalty_kernel(
   }
 }
 
+// The penalty for one row and a context that the host holds, as a copy: y = x with the tokens of
+// the context penalised.  The tokens travel in the kernel's arguments, so the clone, the cleared
+// bitmap, the upload and the marking pass of the general path (five launches and a copy that the
+// host waits for) become this one launch.  A workgroup owns 2048 tokens, marks those of the
+// context in LDS (each once) and writes its 8 tokens per thread.
+constexpr int PR_MAX = 896;      // 3.5 KB of the 4 KB that a launch's arguments may take
+constexpr int PR_TOKENS = 2048;
+struct PrTokens { int32_t t[PR_MAX]; };
+__global__ __launch_bounds__(256) void penalised_row_kernel(const uint16_t* __restrict__ x,
+                                                            uint16_t* __restrict__ y, int V,
+                                                            PrTokens ctx, int n, float pen) {
+  __shared__ uint32_t mark[PR_TOKENS / 32];
+  const int tid = threadIdx.x, t0 = blockIdx.x * PR_TOKENS, c = t0 / 8 + tid;
+  const bool in = c * 8 < V;   // (V is a multiple of 8)
+  uint4 v = make_uint4(0, 0, 0, 0);
+  if (in) v = reinterpret_cast<const uint4*>(x)[c];
+  if (tid < PR_TOKENS / 32) mark[tid] = 0;
+  __syncthreads();
+  for (int i = tid; i < n; i += 256) {
+    const uint32_t d = (uint32_t)ctx.t[i] - (uint32_t)t0;
+    if (ctx.t[i] >= 0 && d < (uint32_t)PR_TOKENS) atomicOr(&mark[d >> 5], 1u << (d & 31));
+  }
+  __syncthreads();
+  if (!in) return;
+  const uint32_t bits = (mark[tid >> 2] >> (8 * (tid & 3))) & 0xFFu;
+  union { uint4 v; uint16_t h[8]; } u;
+  u.v = v;
+  if (bits) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      if ((bits >> e) & 1u) penalise(&u.h[e], pen);
+  }
+  reinterpret_cast<uint4*>(y)[c] = u.v;
+}
+
 // seen[b] |= {tok[b * tok_stride + i] : i < n} (tokens outside [0, V) ignored).
 __global__ void seen_mark_kernel(uint32_t* __restrict__ seen, int words,
                                  const int32_t* __restrict__ tok, long long tok_stride, int n,
@@ -1289,6 +1326,20 @@ LOLLM_API int lollm_repetition_penalty(void* logits, long long ld, int B, int T,
   hipLaunchKernelGGL(repetition_penalty_kernel, dim3((wmax + 255) / 256, B * T), dim3(256), 0,
                      (hipStream_t)stream, (uint16_t*)logits, ld, T, V, seen, words, extra,
                      extra_stride, n_extra0, penalty);
+  return launch_status();
+}
+
+LOLLM_API int lollm_penalised_row(const void* x, void* y, int V, const int32_t* host_tokens, int n,
+                                  float penalty, void* stream) {
+  if (!x || !y || !host_tokens || V <= 0 || V % 8 || n < 0 || !(penalty > 0.f) || !(penalty < 3.0e38f))
+    return LOLLM_EINVAL;
+  if (((uintptr_t)x | (uintptr_t)y) % 16) return LOLLM_EINVAL;
+  if (n > PR_MAX) return LOLLM_EUNSUPPORTED;
+  PrTokens t;
+  memcpy(t.t, host_tokens, sizeof(int32_t) * n);
+  memset(t.t + n, 0, sizeof(int32_t) * (PR_MAX - n));
+  hipLaunchKernelGGL(penalised_row_kernel, dim3((V + PR_TOKENS - 1) / PR_TOKENS), dim3(256), 0, (hipStream_t)stream,
+                     (const uint16_t*)x, (uint16_t*)y, V, t, n, penalty);
   return launch_status();
 }
 

@@ -10,6 +10,7 @@ over the family's `forward(ids, past) -> (logits, past)`.
 from __future__ import annotations
 
 import itertools
+from array import array
 
 import torch
 
@@ -19,24 +20,43 @@ _draws = itertools.count(1)
 SEED = 0x5EED
 
 
+def _host_ids(prev_ids):
+    """The ids as C ints, or None where only the general path takes them: more than a launch
+    carries, or values that are not plain int32 (the tensor constructor decides on those)."""
+    if not isinstance(prev_ids, (list, tuple, set, range)) or len(prev_ids) > ops.PENALISED_ROW_MAX:
+        return None
+    try:
+        return array("i", prev_ids)
+    except (TypeError, OverflowError):
+        return None
+
+
 def sample_next(logits, temperature, top_k, top_p, repetition_penalty=1.0, prev_ids=None,
                 seed=None, offset=None):
-    """(V,) logits on the device -> int token.  The repetition penalty runs in the
-    lollm_repetition_penalty kernel over the bitmap of set(prev_ids) (generate.py:18-22,
-    bf16 arithmetic as the reference's GPU logits have), on a copy of the row."""
+    """(V,) logits on the device -> int token.  The repetition penalty over set(prev_ids)
+    (generate.py:18-22, bf16 arithmetic as the reference's GPU logits have) is applied to a
+    copy of the row: in one launch that carries the ids (lollm_penalised_row), or for a long
+    context through the bitmap of lollm_repetition_penalty."""
     x = logits.reshape(1, -1)
     V = x.shape[1]
     x = x.to(torch.bfloat16)
-    if x.data_ptr() == logits.data_ptr() or not x.is_contiguous():
+    penalise = repetition_penalty != 1.0 and bool(prev_ids)
+    if not x.is_contiguous() or x.data_ptr() % 16:
         x = x.clone(memory_format=torch.contiguous_format)
-    if repetition_penalty != 1.0 and prev_ids:
-        seen = ops.new_seen(1, V, x.device)
-        ops.seen_mark(seen, torch.tensor(list(prev_ids), dtype=torch.int32, device=x.device), V)
-        ops.repetition_penalty(x, seen, repetition_penalty)
+    if penalise:
+        ids = _host_ids(prev_ids) if V % 8 == 0 and 0.0 < repetition_penalty < 3e38 else None
+        if ids is not None:
+            x = ops.penalised_row(x, ids, repetition_penalty)
+        else:
+            if x.data_ptr() == logits.data_ptr():
+                x = x.clone()
+            seen = ops.new_seen(1, V, x.device)
+            ops.seen_mark(seen, torch.tensor(list(prev_ids), dtype=torch.int32, device=x.device), V)
+            ops.repetition_penalty(x, seen, repetition_penalty)
     off = next(_draws) if offset is None else offset
     tok = ops.sample_rows(x, temperature, top_k or 0, top_p if top_p else 1.0,
                           SEED if seed is None else seed, off)
-    return int(tok[0])
+    return tok.item()
 
 
 @torch.no_grad()

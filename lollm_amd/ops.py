@@ -824,6 +824,21 @@ def seen_mark(seen, tokens, V):
     return seen
 
 
+PENALISED_ROW_MAX = 896
+
+
+def penalised_row(logits, tokens, penalty):
+    """A copy of the contiguous bf16 row `logits` (1, V) with the tokens of `tokens` penalised as
+    repetition_penalty does; tokens: an array('i') on the host, at most PENALISED_ROW_MAX."""
+    _need(logits, "logits", torch.bfloat16)
+    out = torch.empty_like(logits)
+    addr, n = tokens.buffer_info()
+    rc = _lib.lib().lollm_penalised_row(_ptr(logits), _ptr(out), logits.numel(), addr, n, float(penalty),
+                                        _stream())
+    _lib.check(rc, "lollm_penalised_row")
+    return out
+
+
 def repetition_penalty(logits, seen, penalty, extra=None, n_extra0=0):
     """In place on bf16 logits (B, T, V) (or (B, V) = T 1): row (b, t) penalises the tokens
     of seen[b] plus extra[b, :n_extra0 + t] (each once), the reference's

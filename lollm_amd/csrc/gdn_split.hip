@@ -7,16 +7,21 @@
 //   gdn_split_prep   one workgroup per (sequence, v-head, chunk): conv, gating, A, Tm, the q.k
 //                    decay; leaves W, U = Tm diag(beta) V, the decay, q and k^T in memory in
 //                    MFMA-operand order (each later load is one coalesced 1 KB)
-//   gdn_split_scan   one workgroup per (sequence, v-head, 32 value columns): the recurrence
+//   gdn_split_scan   one workgroup per (sequence, v-head, 16 or 32 value columns): the recurrence
 //                    V' = U - W S,  O = diag(rq s e^gc) Q S + decay V',
 //                    S <- e^gc_63 S + K^T diag(rk e^(gc_63 - gc)) V'
-//                    -- 68 MFMAs per wave and chunk against the ~1370 of the whole chunk
+//                    -- 68 MFMAs per wave and chunk (32 columns) against ~1370 of the whole chunk
 //   gdn_split_norm   gated RMSNorm of the core output, in place
 // The scan is a chain of chunks, so its step is kept short: the four waves split the 64 tokens
 // (16 each) for V' and O and the 128 keys (32 each) for the state update, every operand but S
 // and V' comes straight from memory to registers one chunk ahead, S and V' pass through LDS
 // as hi / lo bf16 with two barriers per chunk, and a wave keeps its part of S in fp32
 // registers.
+//
+// What bounds it (1 x 1847 tokens, 32 heads: 543 us walked, 130 here): prep 67 us, 18 us per
+// item at one workgroup per CU (149 KB of LDS) over 3.6 rounds, its barriers and the serial
+// solve; the scan about 58 us, 2 us per chunk of dependent reads, products and barriers; the
+// norm 9 us, bandwidth.
 #include "gdn_chunk_common.h"
 
 namespace lollm {
@@ -215,31 +220,33 @@ __global__ __launch_bounds__(256) void gdn_split_prep_kernel(GsArgs s) {
     }
 }
 
-constexpr int GS_COLS = 32;   // value columns of a scan workgroup
-
+// NU 16-column tiles per workgroup.
+template <int NU>
 __global__ __launch_bounds__(256, 2) void gdn_split_scan_kernel(GsArgs s, int heads) {
+  constexpr int GS_COLS = 16 * NU, GROUPS = GL_DK / GS_COLS;
   __shared__ uint16_t sS[2][GS_COLS][GC_PW];   // S hi, lo [column][key]
   __shared__ uint16_t sV[4][GS_COLS][GC_PN];   // V' hi, lo, diag(rk e^..) V' hi, lo [column][token]
   const GdnLayerArgs& a = s.g;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r16 = lane & 15, g4 = lane >> 4;
-  // the four column groups of a head on one XCD (its L2 then serves three of their four
+  // the column groups of a head on one XCD (its L2 then serves all but the first of their
   // reads of W, q, k^T and the decay)
   const int i = blockIdx.x;
-  const int bh = heads % 8 == 0 ? (i / 32) * 8 + i % 8 : i / 4, cg = heads % 8 == 0 ? (i / 8) % 4 : i % 4;
+  const int bh = heads % 8 == 0 ? (i / (8 * GROUPS)) * 8 + i % 8 : i / GROUPS;
+  const int cg = heads % 8 == 0 ? (i / 8) % GROUPS : i % GROUPS;
   const int b = bh / a.Hv, h = bh % a.Hv, hk = h / (a.Hv / a.Hk);
   constexpr size_t SS = (size_t)GL_DK * GL_DK;
   float* st_io = a.rec + ((size_t)(b * 2 + ((a.rec_half[b] & 1) ^ 1)) * a.Hv + h) * SS;
   const uint8_t* ws = s.ws + (size_t)bh * s.nc * GS_ITEM;
   const uint8_t* wq = s.wsqk + (size_t)(b * a.Hk + hk) * s.nc * GS_QK_ITEM;
 
-  gc_f32x4 st[2][2];   // keys 32 w + 16 c + 4 g4 + j, column 32 cg + 16 u + r16
+  gc_f32x4 st[2][NU];   // keys 32 w + 16 c + 4 g4 + j, column 32 cg + 16 u + r16
   const bool zero = a.fresh && s.c0 == 0;
 #pragma unroll
   for (int c = 0; c < 2; ++c)
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
+    for (int u = 0; u < NU; ++u)
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const float x = st_io[(size_t)(32 * wave + 16 * c + 4 * g4 + j) * GL_DK + GS_COLS * cg + 16 * u + r16];
@@ -261,7 +268,7 @@ __global__ __launch_bounds__(256, 2) void gdn_split_scan_kernel(GsArgs s, int he
 #pragma unroll
     for (int c = 0; c < 2; ++c)
 #pragma unroll
-      for (int u = 0; u < 2; ++u)
+      for (int u = 0; u < NU; ++u)
         split4(st[c][u], &sS[0][16 * u + r16][32 * wave + 16 * c + 4 * g4],
                &sS[1][16 * u + r16][32 * wave + 16 * c + 4 * g4]);
   };
@@ -270,7 +277,7 @@ __global__ __launch_bounds__(256, 2) void gdn_split_scan_kernel(GsArgs s, int he
   // operands of a chunk, loaded one chunk before their use (two made no difference)
   struct {   // W, U, q and the scale of V'
     gc_bf16x8 wh[4], wl[4], qr[4];
-    gc_f32x4 un[2], f7;
+    gc_f32x4 un[NU], f7;
   } f;
   struct {   // k^T, the decay, the scales of O and S
     gc_bf16x8 kr[2][2], ih[2], il[2];
@@ -287,8 +294,8 @@ __global__ __launch_bounds__(256, 2) void gdn_split_scan_kernel(GsArgs s, int he
       f.qr[k] = gc_ld8((const uint16_t*)(q + GS_Q + ((wave * 4 + k) * 64 + lane) * 16));
     }
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
-      f.un[u] = *reinterpret_cast<const gc_f32x4*>(w + GS_U + (((cg * 4 + wave) * 2 + u) * 64 + lane) * 16);
+    for (int u = 0; u < NU; ++u)
+      f.un[u] = *reinterpret_cast<const gc_f32x4*>(w + GS_U + (((cg * NU / 2 * 4 + wave) * 2 + (cg * NU + u) % 2) * 64 + lane) * 16);
     f.f7 = *reinterpret_cast<const gc_f32x4*>(w + GS_SC + 4 * (GC_C + 16 * wave + 4 * g4));
   };
   auto load_second = [&](int c) {
@@ -313,16 +320,16 @@ __global__ __launch_bounds__(256, 2) void gdn_split_scan_kernel(GsArgs s, int he
   for (int c = 0; c < s.nc; ++c) {
     const int cn = min(c + 1, s.nc - 1);
     lds_only_barrier();   // S of this chunk written (and V' of the last one read)
-    gc_f32x4 vn[3][2], ov[2][2];
+    gc_f32x4 vn[3][NU], ov[2][NU];
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
+    for (int u = 0; u < NU; ++u) {
       vn[0][u] = f.un[u];
       vn[1][u] = vn[2][u] = ov[0][u] = ov[1][u] = gc_f32x4{0.f, 0.f, 0.f, 0.f};
     }
 #pragma unroll
     for (int k = 0; k < 4; ++k)
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
+      for (int u = 0; u < NU; ++u) {
         const gc_bf16x8 sh = gc_ld8(&sS[0][16 * u + r16][32 * k + 8 * g4]);
         const gc_bf16x8 sl = gc_ld8(&sS[1][16 * u + r16][32 * k + 8 * g4]);
         vn[0][u] = gc_mma(f.wh[k], sh, vn[0][u]);
@@ -332,7 +339,7 @@ __global__ __launch_bounds__(256, 2) void gdn_split_scan_kernel(GsArgs s, int he
         ov[1][u] = gc_mma(f.qr[k], sl, ov[1][u]);
       }
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
+    for (int u = 0; u < NU; ++u) {
       const gc_f32x4 v = vn[0][u] + (vn[1][u] + vn[2][u]);
       const int col = 16 * u + r16, tok = 16 * wave + 4 * g4;
       split4(v, &sV[0][col][tok], &sV[1][col][tok]);
@@ -343,11 +350,11 @@ __global__ __launch_bounds__(256, 2) void gdn_split_scan_kernel(GsArgs s, int he
 #pragma unroll
     for (int cc = 0; cc < 2; ++cc)
 #pragma unroll
-      for (int u = 0; u < 2; ++u) st[cc][u] *= g.eg;
+      for (int u = 0; u < NU; ++u) st[cc][u] *= g.eg;
 #pragma unroll
     for (int s2 = 0; s2 < 2; ++s2)
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
+      for (int u = 0; u < NU; ++u) {
         const gc_bf16x8 qh = gc_ld8(&sV[2][16 * u + r16][32 * s2 + 8 * g4]);
         const gc_bf16x8 ql = gc_ld8(&sV[3][16 * u + r16][32 * s2 + 8 * g4]);
 #pragma unroll
@@ -358,7 +365,7 @@ __global__ __launch_bounds__(256, 2) void gdn_split_scan_kernel(GsArgs s, int he
       }
     put_state();
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
+    for (int u = 0; u < NU; ++u) {
       ov[0][u] = (ov[0][u] + ov[1][u]) * g.rs;
       ov[1][u] = gc_f32x4{0.f, 0.f, 0.f, 0.f};
     }
@@ -366,7 +373,7 @@ __global__ __launch_bounds__(256, 2) void gdn_split_scan_kernel(GsArgs s, int he
     for (int s2 = 0; s2 < 2; ++s2)
       if (s2 <= (wave >> 1)) {
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
+        for (int u = 0; u < NU; ++u) {
           const gc_bf16x8 vh = gc_ld8(&sV[0][16 * u + r16][32 * s2 + 8 * g4]);
           const gc_bf16x8 vl = gc_ld8(&sV[1][16 * u + r16][32 * s2 + 8 * g4]);
           ov[0][u] = gc_mma(g.ih[s2], vh, ov[0][u]);
@@ -380,7 +387,7 @@ __global__ __launch_bounds__(256, 2) void gdn_split_scan_kernel(GsArgs s, int he
       const int t = (s.c0 + c) * GC_C + 16 * wave + 4 * g4 + j;
       if (t < a.T) {
 #pragma unroll
-        for (int u = 0; u < 2; ++u)
+        for (int u = 0; u < NU; ++u)
           outp[(size_t)t * a.value_dim + 16 * u] = gc_bits((__bf16)(ov[0][u][j] + ov[1][u][j]));
       }
     }
@@ -388,7 +395,7 @@ __global__ __launch_bounds__(256, 2) void gdn_split_scan_kernel(GsArgs s, int he
 #pragma unroll
   for (int c = 0; c < 2; ++c)
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
+    for (int u = 0; u < NU; ++u)
 #pragma unroll
       for (int j = 0; j < 4; ++j)
         st_io[(size_t)(32 * wave + 16 * c + 4 * g4 + j) * GL_DK + GS_COLS * cg + 16 * u + r16] = st[c][u][j];
@@ -470,7 +477,14 @@ LOLLM_API int lollm_gdn_layer_split(const void* proj, long long proj_stride, con
     s.nc = nch - s.c0 < seg ? nch - s.c0 : seg;
     hipLaunchKernelGGL(gdn_split_prep_kernel, dim3(heads * s.nc), dim3(256), 0, st, s);
     if ((rc = launch_status())) return rc;
-    hipLaunchKernelGGL(gdn_split_scan_kernel, dim3(heads * (GL_DK / GS_COLS)), dim3(256), 0, st, s, heads);
+    // 16 columns a workgroup where that is still one workgroup per CU (us of the call, 16 / 32
+    // columns: 32 heads x 29 chunks 130 / 145, 16 heads 92 / 107; 64 heads x 24 171 / 170, 96
+    // heads 290 / 273, where the repeated reads of W, q and k^T cost more than the shorter step
+    // gives)
+    if (heads <= 32)
+      hipLaunchKernelGGL(gdn_split_scan_kernel<1>, dim3(heads * 8), dim3(256), 0, st, s, heads);
+    else
+      hipLaunchKernelGGL(gdn_split_scan_kernel<2>, dim3(heads * 4), dim3(256), 0, st, s, heads);
     if ((rc = launch_status())) return rc;
   }
   hipLaunchKernelGGL(gdn_split_norm_kernel, dim3(B * T, (Hv + 15) / 16), dim3(256), 0, st, s.g);

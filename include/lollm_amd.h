@@ -377,10 +377,13 @@ int lollm_gdn_layer_split(const void* proj, long long proj_stride, const void* c
 /* C = A W^T (bf16, fp32 sums) for many rows, W from lollm_gemm_tile_weights with the same
  * epilogue: 0 C is (M, N); 1 W = [gate; up], C is (M, N / 2) = silu(gate) * up with
  * lollm_gemm's rounding points.  tile: the output tile of a workgroup as 10 x rows / 64 +
- * columns / 64, one of 44, 34, 43, 24 (it changes the time only).  N a multiple of 64, K of
- * 128, lda and ldc of 8; A, Wt and C 16-byte aligned. */
+ * columns / 64, one of 44, 34, 43, 24 (it changes the time only).  splits: parts of K (tile 24
+ * only, a divisor of K / 128) whose fp32 sums go through the workspace of splits x M x N x 4
+ * bytes and are added in k order; 1 for none (workspace unused).  N a multiple of 64, K of
+ * 128, lda and ldc of 8; A, Wt, C and workspace 16-byte aligned. */
 int lollm_gemm_rows(const void* A, long long lda, const void* Wt, void* C, long long ldc, int M,
-                    int N, int K, int epilogue, int tile, void* stream);
+                    int N, int K, int epilogue, int tile, int splits, void* workspace,
+                    long long workspace_bytes, void* stream);
 
 /* Greedy acceptance (temperature 0) without the verify logits: argmax (B, k + 1) int32
  * holds the argmax token of each verify row (lollm_gemm_argmax on the lm_head, same

@@ -68,8 +68,8 @@ SIGNATURES = {
     "lollm_gemm_workspace_bytes": ([_I, _I, _I, _I], ctypes.c_longlong),
     "lollm_gemm": ([_P, ctypes.c_longlong, _P, _P, ctypes.c_longlong, _I, _I, _I, _I, _P,
                     ctypes.c_longlong, _I, _P], _I),
-    "lollm_gemm_rows": ([_P, ctypes.c_longlong, _P, _P, ctypes.c_longlong, _I, _I, _I, _I, _I, _P],
-                        _I),
+    "lollm_gemm_rows": ([_P, ctypes.c_longlong, _P, _P, ctypes.c_longlong, _I, _I, _I, _I, _I, _I, _P,
+                         ctypes.c_longlong, _P], _I),
     "lollm_gemm_rowmax_slots": ([_I], _I),
     "lollm_gemm_logits": ([_P, ctypes.c_longlong, _P, _I, _I, _I, _P, ctypes.c_longlong, _P,
                            ctypes.c_longlong, _P, _I, _P, _I, _I, _I, _F, _P, ctypes.c_longlong,

@@ -35,6 +35,8 @@ struct GrArgs {
   long long lda, ldc;
   int M, N, K;
   int mt, nt;           // tiles
+  float* part;          // split K: (splits, M, N) fp32
+  int splits;
 };
 
 __device__ __forceinline__ float gr_round(float x) { return (float)(__bf16)x; }
@@ -65,7 +67,8 @@ template <int N, int MORE> __device__ __forceinline__ void gr_wait_if(int more) 
 // keeps an accumulator in the accumulator registers
 __device__ __forceinline__ void gr_pin(gr_f32x4& v) { asm volatile("" : "+a"(v)); }
 
-template <int MT, int NT, bool SWIGLU>
+// SPLIT: K in a.splits equal parts, a (tile, part) to a workgroup, fp32 sums to a.part.
+template <int MT, int NT, bool SWIGLU, bool SPLIT>
 __device__ __forceinline__ void gr_tiles(const GrArgs& a) {
   constexpr int BM = 64 * MT, BN = 64 * NT;
   constexpr int ABYTES = BM * 128, BBYTES = BN * 64;   // rows of a k64 pair, columns of a k32 step
@@ -76,24 +79,29 @@ __device__ __forceinline__ void gr_tiles(const GrArgs& a) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r16 = lane & 15, g4 = lane >> 4;
   const int wm = wave & 1, wn = wave >> 1;
-  const int ntiles = a.mt * a.nt;
+  const int ntiles = a.mt * a.nt * (SPLIT ? a.splits : 1);
 
   // Tile number v = blockIdx.x + i gridDim.x: an XCD (workgroups i, i + 8, ..) takes a
   // contiguous run of the tiles, ordered in bands of 8 row tiles, so that the 32 tiles it works
   // on at a time share rows and columns in its L2.
-  auto locate = [&](int v, int& m0, int& n0) {
-    const int x = v & 7, t = x * (ntiles / 8) + min(x, ntiles % 8) + (v >> 3);
+  auto locate = [&](int v, int& m0, int& n0, int& part) {
+    const int x = v & 7, u = x * (ntiles / 8) + min(x, ntiles % 8) + (v >> 3);
+    // (the row tiles of a column tile's part next to each other: they read the same W)
+    const int tiles = a.mt * a.nt, t = SPLIT ? u % tiles : u;
+    part = SPLIT ? u / tiles : 0;
     const int band = t / (8 * a.nt), r = t - band * 8 * a.nt, hb = min(8, a.mt - 8 * band);
     m0 = (8 * band + r % hb) * BM;
     n0 = (r / hb) * BN;
   };
   // descriptors of a tile's rows of A and blocks of W: what lies past M or N reads as zero
-  auto rsrc_a = [&](int m0, bool live) {
-    return buf_rsrc(a.A + (live ? (size_t)m0 * a.lda : 0),
-                    live ? (uint32_t)(min(BM, a.M - m0) - 1) * (uint32_t)(2 * a.lda) + 2u * a.K : 0u);
+  const int kpart = SPLIT ? a.K / a.splits : a.K;   // k of a part: a multiple of 128
+  auto rsrc_a = [&](int m0, int part, bool live) {
+    return buf_rsrc(a.A + (live ? (size_t)m0 * a.lda + (size_t)part * kpart : 0),
+                    live ? (uint32_t)(min(BM, a.M - m0) - 1) * (uint32_t)(2 * a.lda) + 2u * kpart : 0u);
   };
-  auto rsrc_b = [&](int n0, bool live) {
-    return buf_rsrc(a.Wt + (live ? (size_t)n0 * a.K : 0), live ? (uint32_t)(min(BN, a.N - n0) / 16) * (32u * a.K) : 0u);
+  auto rsrc_b = [&](int n0, int part, bool live) {
+    return buf_rsrc(a.Wt + (live ? (size_t)n0 * a.K + (size_t)part * kpart * 16 : 0),
+                    live ? (uint32_t)(min(BN, a.N - n0) / 16 - 1) * (32u * a.K) + 32u * kpart : 0u);
   };
   // Loads: A for a pair of steps, 8 rows of 128 bytes (whole cache lines) per instruction (lane:
   // row lane / 8, chunk lane % 8 of the place written, whose source chunk undoes the swizzle);
@@ -121,10 +129,10 @@ __device__ __forceinline__ void gr_tiles(const GrArgs& a) {
   };
   auto read_b = [&](const unsigned char* s, int j) { return *reinterpret_cast<const gr_bf16x8*>(s + br + 1024 * j); };
 
-  const int steps = a.K / 32;   // a multiple of 4
-  int v = blockIdx.x, m0, n0;
-  locate(v, m0, n0);
-  __amdgpu_buffer_rsrc_t ars = rsrc_a(m0, true), brs = rsrc_b(n0, true);
+  const int steps = kpart / 32;   // a multiple of 4
+  int v = blockIdx.x, m0, n0, part;
+  locate(v, m0, n0, part);
+  __amdgpu_buffer_rsrc_t ars = rsrc_a(m0, part, true), brs = rsrc_b(n0, part, true);
   auto fill_a = [&](unsigned char* s, int k) {
 #pragma unroll
     for (int i = 0; i < AI; ++i) dma_a(s, ars, i, 64u * k);
@@ -148,7 +156,7 @@ __device__ __forceinline__ void gr_tiles(const GrArgs& a) {
 
   constexpr int OC = SWIGLU ? 16 * NT : 32 * NT;     // output columns of a wave
   constexpr int PER = OC / 8;                        // 16-byte chunks per row of it
-  constexpr int STORES = MT * (32 * PER / 64);       // store instructions of a wave's epilogue
+  constexpr int STORES = SPLIT ? AF * BF : MT * (32 * PER / 64);   // store instructions of a wave's epilogue
   static_assert(AI + BI + STORES <= 63, "vmcnt");
   int after = 0;   // a tile came before this one
 
@@ -156,9 +164,9 @@ __device__ __forceinline__ void gr_tiles(const GrArgs& a) {
     // the next tile, whose first steps follow this one's last
     const int vn = v + (int)gridDim.x;
     const bool more = vn < ntiles;
-    int m1 = 0, n1 = 0;
-    if (more) locate(vn, m1, n1);
-    const __amdgpu_buffer_rsrc_t arn = rsrc_a(m1, more), brn = rsrc_b(n1, more);
+    int m1 = 0, n1 = 0, part1 = 0;
+    if (more) locate(vn, m1, n1, part1);
+    const __amdgpu_buffer_rsrc_t arn = rsrc_a(m1, part1, more), brn = rsrc_b(n1, part1, more);
 
     gr_f32x4 acc[BF][AF];
 #pragma unroll
@@ -213,59 +221,78 @@ __device__ __forceinline__ void gr_tiles(const GrArgs& a) {
 #pragma unroll
       for (int i = 0; i < AF; ++i) gr_pin(acc[j][i]);
 
-    // Epilogue per SR rows: the accumulators (lane: row r16, columns 16 j + 4 g4 + e) through the
-    // wave's quarter of b3 (free: its last data was read before the last barrier, and the next
-    // DMA into it follows the next one) as bf16, 16-byte chunk c of row r at c ^ (r & XM), then
-    // 16-byte stores along the rows, dropped past M and N by the descriptor (every store is
-    // issued: the waits above count them).
-    constexpr int PITCH = 2 * OC, SR = SWIGLU ? 32 : 16;   // rows staged at a time
-    constexpr int XM = PER % 8 == 0 ? 7 : (PER % 4 == 0 ? 3 : 1);
-    static_assert(SR * PITCH <= BBYTES / 4, "staging");
-    unsigned char* st = b3 + wave * (BBYTES / 4);
-    const int nout = SWIGLU ? a.N / 2 : a.N, c0 = (SWIGLU ? n0 / 2 : n0) + OC * wn;
-    const __amdgpu_buffer_rsrc_t crs = buf_rsrc(
-        a.C + (size_t)m0 * a.ldc, (uint32_t)(min(BM, a.M - m0) - 1) * (uint32_t)(2 * a.ldc) + 2u * nout);
-    // (from an opaque copy of the lane, so that no address is kept through the products)
-    int elane = lane;
-    asm volatile("" : "+v"(elane));
-    const int er16 = elane & 15, eg4 = elane >> 4;
+    if constexpr (SPLIT) {
+      // the part's sums as they are: 4 columns of a row per lane
+      int elane = lane;
+      asm volatile("" : "+v"(elane));
+      const int er16 = elane & 15, eg4 = elane >> 4;
+      const __amdgpu_buffer_rsrc_t prs = buf_rsrc(a.part + ((size_t)part * a.M + m0) * a.N,
+                                                  (uint32_t)min(BM, a.M - m0) * (uint32_t)(4 * a.N));
 #pragma unroll
-    for (int i = 0; i < 32 * MT / SR; ++i) {
+      for (int i = 0; i < AF; ++i)
 #pragma unroll
-      for (int u = 0; u < SR / 16; ++u)
-#pragma unroll
-        for (int j = 0; j < BF; j += SWIGLU ? 2 : 1) {
-          gr_f32x4 y = acc[j][SR / 16 * i + u];
-          int col = 16 * j + 4 * eg4;
-          if constexpr (SWIGLU) {
-            // a block holds 8 gate rows, then their 8 up rows, lanes 32 apart: the swap gives the
-            // lower lanes block j's pairs and the upper ones block j + 1's
-            const gr_f32x4 t = acc[j + 1][SR / 16 * i + u];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(y[e]), __float_as_uint(t[e]), false, false);
-              y[e] = gr_silu_bf16(__uint_as_float(sw[0])) * gr_round(__uint_as_float(sw[1]));
-            }
-            col = 8 * (j + (eg4 >> 1)) + 4 * (eg4 & 1);
-          }
-          *reinterpret_cast<gr_u32x2*>(st + (16 * u + er16) * PITCH + ((2 * col) ^ (16 * (er16 & XM)))) =
-              gr_u32x2{gr_pack(y[0], y[1]), gr_pack(y[2], y[3])};
+        for (int j = 0; j < BF; ++j) {
+          const int row = 32 * MT * wm + 16 * i + er16, col = n0 + 32 * NT * wn + 16 * j + 4 * eg4;
+          const uint32_t off = col < a.N ? (uint32_t)row * (uint32_t)(4 * a.N) + 4u * col : 0xfffffff0u;
+          const gr_f32x4 t = acc[j][i];
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, t), prs, off, 0, 0);
         }
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the wave's own staging
+    } else {
+      // Epilogue per SR rows: the accumulators (lane: row r16, columns 16 j + 4 g4 + e) through the
+      // wave's quarter of b3 (free: its last data was read before the last barrier, and the next
+      // DMA into it follows the next one) as bf16, 16-byte chunk c of row r at c ^ (r & XM), then
+      // 16-byte stores along the rows, dropped past M and N by the descriptor (every store is
+      // issued: the waits above count them).
+      constexpr int PITCH = 2 * OC, SR = SWIGLU ? 32 : 16;   // rows staged at a time
+      constexpr int XM = PER % 8 == 0 ? 7 : (PER % 4 == 0 ? 3 : 1);
+      static_assert(SR * PITCH <= BBYTES / 4, "staging");
+      unsigned char* st = b3 + wave * (BBYTES / 4);
+      const int nout = SWIGLU ? a.N / 2 : a.N, c0 = (SWIGLU ? n0 / 2 : n0) + OC * wn;
+      const __amdgpu_buffer_rsrc_t crs = buf_rsrc(
+          a.C + (size_t)m0 * a.ldc, (uint32_t)(min(BM, a.M - m0) - 1) * (uint32_t)(2 * a.ldc) + 2u * nout);
+      // (from an opaque copy of the lane, so that no address is kept through the products)
+      int elane = lane;
+      asm volatile("" : "+v"(elane));
+      const int er16 = elane & 15, eg4 = elane >> 4;
 #pragma unroll
-      for (int n = 0; n < SR * PER / 64; ++n) {
-        const int c = 64 * n + elane, r = c / PER, cc = c % PER;
-        const int row = 32 * MT * wm + SR * i + r, col = c0 + 8 * cc;
-        const u32x4_t w = *reinterpret_cast<const u32x4_t*>(st + r * PITCH + 16 * (cc ^ (r & XM)));
-        const uint32_t off = col < nout ? (uint32_t)row * (uint32_t)(2 * a.ldc) + 2u * col : 0xfffffff0u;
-        __builtin_amdgcn_raw_buffer_store_b128(w, crs, off, 0, 0);
+      for (int i = 0; i < 32 * MT / SR; ++i) {
+#pragma unroll
+        for (int u = 0; u < SR / 16; ++u)
+#pragma unroll
+          for (int j = 0; j < BF; j += SWIGLU ? 2 : 1) {
+            gr_f32x4 y = acc[j][SR / 16 * i + u];
+            int col = 16 * j + 4 * eg4;
+            if constexpr (SWIGLU) {
+              // a block holds 8 gate rows, then their 8 up rows, lanes 32 apart: the swap gives the
+              // lower lanes block j's pairs and the upper ones block j + 1's
+              const gr_f32x4 t = acc[j + 1][SR / 16 * i + u];
+#pragma unroll
+              for (int e = 0; e < 4; ++e) {
+                const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(y[e]), __float_as_uint(t[e]), false, false);
+                y[e] = gr_silu_bf16(__uint_as_float(sw[0])) * gr_round(__uint_as_float(sw[1]));
+              }
+              col = 8 * (j + (eg4 >> 1)) + 4 * (eg4 & 1);
+            }
+            *reinterpret_cast<gr_u32x2*>(st + (16 * u + er16) * PITCH + ((2 * col) ^ (16 * (er16 & XM)))) =
+                gr_u32x2{gr_pack(y[0], y[1]), gr_pack(y[2], y[3])};
+          }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the wave's own staging
+#pragma unroll
+        for (int n = 0; n < SR * PER / 64; ++n) {
+          const int c = 64 * n + elane, r = c / PER, cc = c % PER;
+          const int row = 32 * MT * wm + SR * i + r, col = c0 + 8 * cc;
+          const u32x4_t w = *reinterpret_cast<const u32x4_t*>(st + r * PITCH + 16 * (cc ^ (r & XM)));
+          const uint32_t off = col < nout ? (uint32_t)row * (uint32_t)(2 * a.ldc) + 2u * col : 0xfffffff0u;
+          __builtin_amdgcn_raw_buffer_store_b128(w, crs, off, 0, 0);
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       }
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     }
     if (!more) break;
     v = vn;
     m0 = m1;
     n0 = n1;
+    part = part1;
     ars = arn;
     brs = brn;
   }
@@ -273,9 +300,38 @@ __device__ __forceinline__ void gr_tiles(const GrArgs& a) {
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
-template <int MT, int NT, bool SWIGLU>
+template <int MT, int NT, bool SWIGLU, bool SPLIT>
 __global__ __launch_bounds__(GR_THREADS, 1) void gemm_rows_kernel(GrArgs a) {
-  gr_tiles<MT, NT, SWIGLU>(a);   // (a device function: the host pass drops the kernel's stub otherwise)
+  gr_tiles<MT, NT, SWIGLU, SPLIT>(a);   // (a device function: the host pass drops the kernel's stub otherwise)
+}
+
+// C from the parts, added in k order: 8 columns of C per thread.
+template <bool SWIGLU>
+__global__ __launch_bounds__(256) void gemm_rows_reduce_kernel(GrArgs a) {
+  const int per = (SWIGLU ? a.N / 2 : a.N) / 8;
+  const long long c = (long long)blockIdx.x * 256 + threadIdx.x;
+  if (c >= (long long)a.M * per) return;
+  const int row = (int)(c / per), cc = (int)(c % per);
+  const float* p = a.part + (size_t)row * a.N + (SWIGLU ? 16 : 8) * cc;
+  constexpr int Q = SWIGLU ? 4 : 2;
+  gr_f32x4 s[Q];
+#pragma unroll
+  for (int q = 0; q < Q; ++q) s[q] = reinterpret_cast<const gr_f32x4*>(p)[q];
+  for (int n = 1; n < a.splits; ++n) {
+    p += (size_t)a.M * a.N;
+#pragma unroll
+    for (int q = 0; q < Q; ++q) s[q] += reinterpret_cast<const gr_f32x4*>(p)[q];
+  }
+  u32x4_t w;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int q = e >> 1, l = 2 * (e & 1);
+    if (SWIGLU)   // 8 gate columns, then their 8 up columns
+      w[e] = gr_pack(gr_silu_bf16(s[q][l]) * gr_round(s[2 + q][l]), gr_silu_bf16(s[q][l + 1]) * gr_round(s[2 + q][l + 1]));
+    else
+      w[e] = gr_pack(s[q][l], s[q][l + 1]);
+  }
+  *reinterpret_cast<u32x4_t*>(a.C + (size_t)row * a.ldc + 8 * cc) = w;
 }
 
 template <bool SWIGLU>
@@ -286,11 +342,19 @@ static int gr_launch(GrArgs& a, int tile, int cus, hipStream_t st) {
   const long long n = (long long)a.mt * a.nt;
   if (n > 0x3fffffff) return LOLLM_EUNSUPPORTED;
   const dim3 g((unsigned)(n < cus ? n : cus)), b(GR_THREADS);
+  if (a.splits > 1) {
+    const long long u = n * a.splits, chunks = (long long)a.M * (SWIGLU ? a.N / 2 : a.N) / 8;
+    hipLaunchKernelGGL((gemm_rows_kernel<2, 4, false, true>), dim3((unsigned)(u < cus ? u : cus)), b, 0, st, a);
+    const int rc = launch_status();
+    if (rc) return rc;
+    hipLaunchKernelGGL(gemm_rows_reduce_kernel<SWIGLU>, dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0, st, a);
+    return launch_status();
+  }
   switch (tile) {
-    case 44: hipLaunchKernelGGL((gemm_rows_kernel<4, 4, SWIGLU>), g, b, 0, st, a); break;
-    case 34: hipLaunchKernelGGL((gemm_rows_kernel<3, 4, SWIGLU>), g, b, 0, st, a); break;
-    case 43: hipLaunchKernelGGL((gemm_rows_kernel<4, 3, SWIGLU>), g, b, 0, st, a); break;
-    case 24: hipLaunchKernelGGL((gemm_rows_kernel<2, 4, SWIGLU>), g, b, 0, st, a); break;
+    case 44: hipLaunchKernelGGL((gemm_rows_kernel<4, 4, SWIGLU, false>), g, b, 0, st, a); break;
+    case 34: hipLaunchKernelGGL((gemm_rows_kernel<3, 4, SWIGLU, false>), g, b, 0, st, a); break;
+    case 43: hipLaunchKernelGGL((gemm_rows_kernel<4, 3, SWIGLU, false>), g, b, 0, st, a); break;
+    case 24: hipLaunchKernelGGL((gemm_rows_kernel<2, 4, SWIGLU, false>), g, b, 0, st, a); break;
     default: return LOLLM_EINVAL;
   }
   return launch_status();
@@ -301,13 +365,17 @@ static int gr_launch(GrArgs& a, int tile, int cus, hipStream_t st) {
 using namespace lollm;
 
 LOLLM_API int lollm_gemm_rows(const void* A, long long lda, const void* Wt, void* C, long long ldc, int M, int N,
-                              int K, int epilogue, int tile, void* stream) {
+                              int K, int epilogue, int tile, int splits, void* workspace,
+                              long long workspace_bytes, void* stream) {
   if (!A || !Wt || !C) return LOLLM_EINVAL;
   if (M <= 0 || N <= 0 || K <= 0 || lda < K || epilogue < 0 || epilogue > 1) return LOLLM_EINVAL;
   if (N % 64 || K % 128 || lda % 8 || ldc % 8 || ldc < (epilogue ? N / 2 : N)) return LOLLM_EINVAL;
-  if (((uintptr_t)A | (uintptr_t)Wt | (uintptr_t)C) % 16) return LOLLM_EINVAL;
+  if (((uintptr_t)A | (uintptr_t)Wt | (uintptr_t)C | (uintptr_t)workspace) % 16) return LOLLM_EINVAL;
+  if (splits < 1 || K / 128 % splits || (splits > 1 && tile != 24)) return LOLLM_EINVAL;
+  if (splits > 1 && (!workspace || workspace_bytes < 4LL * splits * M * N)) return LOLLM_EINVAL;
   // 32-bit byte offsets inside a tile
-  if (256LL * 2 * lda >= (1LL << 31) || 256LL * 2 * ldc >= (1LL << 31) || 256LL * 2 * K >= (1LL << 31))
+  if (256LL * 2 * lda >= (1LL << 31) || 256LL * 2 * ldc >= (1LL << 31) || 256LL * 2 * K >= (1LL << 31) ||
+      256LL * 4 * N >= (1LL << 31))
     return LOLLM_EUNSUPPORTED;
   int dev = 0, cus = 0;
   if (hipGetDevice(&dev) != hipSuccess) return LOLLM_EUNSUPPORTED;
@@ -316,6 +384,7 @@ LOLLM_API int lollm_gemm_rows(const void* A, long long lda, const void* Wt, void
   GrArgs a;
   a.A = (const uint16_t*)A; a.Wt = (const uint16_t*)Wt; a.C = (uint16_t*)C;
   a.lda = lda; a.ldc = ldc; a.M = M; a.N = N; a.K = K;
+  a.part = (float*)workspace; a.splits = splits;
   return epilogue ? gr_launch<true>(a, tile, cus, (hipStream_t)stream)
                   : gr_launch<false>(a, tile, cus, (hipStream_t)stream);
 }

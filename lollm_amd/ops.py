@@ -279,9 +279,10 @@ def gemm_rows_tile(M, N, K, epilogue, cus):
     that is not full runs each step faster).
     Too few tiles leave CUs idle, where the library splits K: from 0.6 of the CUs on this
     kernel is as fast (N = 4096, rows: 1024 0.77 of the library's speed, 1536 0.94 - 1.04, 1847
-    1.05 - 1.12).  One full round of 256 x 256 tiles is the library's best case (N = 4096, 3998
-    rows: 0.97); everywhere else its rounds are less even (4500 rows 1.0 - 1.9, N = 12352 1.0 -
-    1.65, N = 18432 0.98 - 1.36)."""
+    1.05 - 1.12; N = 18432, 200 rows 0.96, 320 1.06), with few columns (N < 4096: short calls
+    of a small model) from one per CU on.  One full round of 256 x 256 tiles is the library's
+    best case (N = 4096, 3998 rows: 0.97); everywhere else its rounds are less even (4500 rows
+    1.0 - 1.9, N = 12352 1.0 - 1.65, N = 18432 0.98 - 1.36)."""
     best, tile, count = None, 0, 0
     for t, us in GEMM_ROWS_STEP_US.items():
         n = -(-M // (64 * (t // 10))) * -(-N // (64 * (t % 10)))
@@ -289,7 +290,7 @@ def gemm_rows_tile(M, N, K, epilogue, cus):
         cost = (n // cus + (0.72 + 0.28 * part if part else 0.0)) * (K // 32 + GEMM_ROWS_EPILOGUE_STEPS) * us
         if best is None or cost < best:
             best, tile, count = cost, t, n
-    if 10 * count < 6 * cus:
+    if 10 * count < (6 if N >= 4096 else 10) * cus:
         return 0
     whole = -(-M // 256) * -(-N // 256)
     if epilogue == GEMM_NONE and 100 * whole >= 93 * cus and whole <= cus:
@@ -297,9 +298,27 @@ def gemm_rows_tile(M, N, K, epilogue, cus):
     return tile
 
 
-def gemm_rows(x, tiled, N, K, epilogue, tile):
+@functools.lru_cache(maxsize=4096)
+def gemm_rows_splits(M, N, K, epilogue, cus):
+    """Parts of K for a product whose tiles leave most CUs idle, or 1 for the library: as many as
+    still give one (128 x 256 tile, part) per CU.  Worth the fp32 parts and the second launch
+    from four parts of a long K on (N = 4096, us, library / here: K = 12288, 96 rows 42 / 27,
+    200 39 / 34, 400 66 / 48, 512 65 / 59; K = 8192, 128 rows 43 / 27, 512 53 / 46; two parts
+    700 rows 58 / 69; K = 4096, 256 rows 20 / 24)."""
+    if K < 8192 or epilogue != GEMM_NONE:
+        return 1
+    tiles = -(-M // 128) * -(-N // 256)
+    best = 1
+    for s in range(4, cus // max(tiles, 1) + 1):
+        if (K // 128) % s == 0:
+            best = s
+    return best
+
+
+def gemm_rows(x, tiled, N, K, epilogue, tile, splits=1):
     """y = x W^T for many rows x (..., K) bf16; `tiled` from gemm_tile_weights with the same
-    epilogue (GEMM_SWIGLU: silu(gate) * up), tile from gemm_rows_tile."""
+    epilogue (GEMM_SWIGLU: silu(gate) * up), tile from gemm_rows_tile or splits (with tile 24)
+    from gemm_rows_splits."""
     M = x.numel() // K
     if x.shape[-1] != K:
         raise ValueError(f"x has {x.shape[-1]} features, expected {K}")
@@ -308,8 +327,10 @@ def gemm_rows(x, tiled, N, K, epilogue, tile):
     _need(tiled, "tiled", torch.bfloat16, (N * K,))
     oc = N // 2 if epilogue == GEMM_SWIGLU else N
     out = torch.empty(*x.shape[:-1], oc, dtype=torch.bfloat16, device=x.device)
-    rc = _lib.lib().lollm_gemm_rows(_ptr(x), K, _ptr(tiled), _ptr(out), oc, M, N, K, epilogue, tile,
-                                    _stream())
+    need = 4 * splits * M * N if splits > 1 else 0
+    ws = torch.empty(need, dtype=torch.uint8, device=x.device) if need else None
+    rc = _lib.lib().lollm_gemm_rows(_ptr(x), K, _ptr(tiled), _ptr(out), oc, M, N, K, epilogue, tile, splits,
+                                    _ptr(ws), need, _stream())
     _lib.check(rc, "lollm_gemm_rows")
     return out
 

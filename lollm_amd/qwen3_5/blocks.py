@@ -7,7 +7,7 @@ q|k|v, MLP gate|up), so a layer issues 4 GEMMs plus fused HIP kernels for everyt
 between them.  A GEMM over at most 64 rows (the verify and draft passes) streams a
 tiled copy of its weight through lollm_gemm, with SiLU(gate) * up fused into the
 gate|up GEMM; longer calls (the prefill) take lollm_gemm_rows on the same copy, SwiGLU
-fused too, where its tiles fill the chip, else hipBLASLt on the row-major weight.
+fused too, where its tiles (or its parts of a long K) fill the chip, else hipBLASLt on the row-major weight.
 """
 
 from __future__ import annotations
@@ -90,13 +90,18 @@ class Projection:
     def path(self, rows):
         return gemm_path(self.N, self.K, self.epilogue, rows, self.tiled is not None)
 
-    def rows_tile(self, x, rows):
-        """The lollm_gemm_rows tile of a call past the few-row GEMM, 0 for hipBLASLt: a pure
-        function of the shape (and 0 where only F.linear serves: another dtype, a gradient)."""
+    def rows_plan(self, x, rows):
+        """(tile, K parts) of lollm_gemm_rows for a call past the few-row GEMM, tile 0 for
+        hipBLASLt: a pure function of the shape (and 0 where only F.linear serves: another
+        dtype, a gradient)."""
         if (self.tiled is None or x.dtype != torch.bfloat16 or not x.is_cuda
                 or x.data_ptr() % 16 or (x.requires_grad and torch.is_grad_enabled())):
-            return 0
-        return ops.gemm_rows_tile(rows, self.N, self.K, self.epilogue, _cus())
+            return 0, 1
+        tile = ops.gemm_rows_tile(rows, self.N, self.K, self.epilogue, _cus())
+        if tile:
+            return tile, 1
+        splits = ops.gemm_rows_splits(rows, self.N, self.K, self.epilogue, _cus())
+        return (24, splits) if splits > 1 else (0, 1)
 
     def argmax_grid(self, rows):
         """Workgroups of the fused lm_head argmax (lollm_gemm_argmax): one per CU."""
@@ -109,9 +114,9 @@ class Projection:
     def __call__(self, x):
         rows = x.numel() // self.K
         if self.path(rows) == "blas":
-            tile = self.rows_tile(x, rows)
+            tile, splits = self.rows_plan(x, rows)
             if tile:
-                return ops.gemm_rows(x, self.tiled, self.N, self.K, self.epilogue, tile)
+                return ops.gemm_rows(x, self.tiled, self.N, self.K, self.epilogue, tile, splits)
             return self._blas(x)
         return ops.gemm(x, self.tiled, self.N, self.K, self.epilogue, grid=self.grid(rows))
 

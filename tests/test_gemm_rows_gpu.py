@@ -29,7 +29,7 @@ def test_gemm_rows_matches_fp32(M, N, K, tile):
     out = torch.full((M + 1, N), 7.0, dtype=torch.bfloat16, device="cuda")
     from lollm_amd import _lib
     xd = x.cuda()
-    rc = _lib.lib().lollm_gemm_rows(xd.data_ptr(), K, t.data_ptr(), out.data_ptr(), N, M, N, K, 0, tile,
+    rc = _lib.lib().lollm_gemm_rows(xd.data_ptr(), K, t.data_ptr(), out.data_ptr(), N, M, N, K, 0, tile, 1, None, 0,
                                     torch.cuda.current_stream().cuda_stream)
     assert rc == 0
     close(out[:M], x.float() @ W.float().t())
@@ -74,11 +74,46 @@ def test_projection_takes_the_rows_kernel_and_keeps_gradients():
     x, W = case(1200, 8192, 256, seed=4)
     p = Projection(W.cuda())
     xd = x.cuda()
-    assert p.rows_tile(xd, 1200) and not p.rows_tile(xd.float(), 1200)
+    assert p.rows_plan(xd, 1200)[0] and not p.rows_plan(xd.float(), 1200)[0]
     close(p(xd), x.float() @ W.float().t())
     xg = xd.clone().requires_grad_()
     p(xg).float().sum().backward()
     assert xg.grad is not None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,splits,epi", [(65, 320, 1536, 12, 0), (129, 256, 512, 4, 0), (257, 1088, 384, 3, 0),
+                                              (96, 4096, 8192, 16, 0), (100, 448, 256, 2, 1), (300, 8192, 256, 2, 0)])
+def test_gemm_rows_split_k(M, N, K, splits, epi):
+    """K in parts: each part's fp32 sums added in order, one rounding at the end.  The last case
+    has more (tile, part) pairs than CUs."""
+    from lollm_amd import ops
+    print(f"case gemm rows split M={M} N={N} K={K} splits={splits} epi={epi}", flush=True)
+    x, W = case(M, N, K, seed=M + K)
+    W, xd = (W.float() * 3).bfloat16().cuda(), x.cuda()
+    got = ops.gemm_rows(xd, ops.gemm_tile_weights(W, epi), N, K, epi, 24, splits)
+    one = ops.gemm_rows(xd, ops.gemm_tile_weights(W, epi), N, K, epi, 24)
+    if not epi:
+        close(got, x.float() @ W.float().cpu().t())
+    # another order of the same fp32 sums: a bf16 rounding (two with SwiGLU) may flip
+    assert (got != one).float().mean() <= 2e-2
+    torch.testing.assert_close(got.float(), one.float(), rtol=2 ** -6, atol=2e-3)
+    from lollm_amd import _lib
+    rc = _lib.lib().lollm_gemm_rows(xd.data_ptr(), K, 16, got.data_ptr(), N, M, N, K, 0, 24, splits, xd.data_ptr(),
+                                    4 * splits * M * N - 1, None)
+    assert rc == 1      # a short workspace is refused before any launch
+
+
+def test_rows_splits_rule():
+    from lollm_amd import ops
+    f = ops.gemm_rows_splits
+    assert f(96, 4096, 12288, 0, 256) == 16 and f(200, 4096, 12288, 0, 256) == 8
+    assert f(512, 4096, 8192, 0, 256) == 4 and f(700, 4096, 8192, 0, 256) == 1
+    assert f(96, 4096, 4096, 0, 256) == 1 and f(96, 24576, 12288, 1, 256) == 1
+    for M in range(65, 3000, 37):
+        for N, K in ((4096, 12288), (4096, 8192), (1024, 8192), (151936, 8192)):
+            s = f(M, N, K, 0, 256)
+            assert (K // 128) % s == 0 and (s == 1 or -(-M // 128) * -(-N // 256) * s <= 256)
 
 
 def test_rows_tile_rule():
@@ -101,8 +136,8 @@ def test_gemm_rows_refuses_bad_arguments():
     """Before any HIP call, so without a device."""
     from lollm_amd import _lib
     f = _lib.lib().lollm_gemm_rows
-    ok = (16, 128, 16, 16, 64, 1, 64, 128, 0, 44, None)
-    for i, v in ((0, None), (2, None), (3, None), (5, 0), (6, 96), (7, 64), (1, 64), (1, 132), (4, 32), (8, 2), (0, 8)):
+    ok = (16, 128, 16, 16, 64, 1, 64, 128, 0, 44, 1, None, 0, None)
+    for i, v in ((0, None), (2, None), (3, None), (5, 0), (6, 96), (7, 64), (1, 64), (1, 132), (4, 32), (8, 2), (0, 8), (10, 0), (10, 2)):
         a = list(ok)
         a[i] = v
         assert f(*a) == 1, (i, v)

@@ -151,7 +151,9 @@ int lollm_spec_accept_noalloc(const void* target, const void* draft, const int32
 /* One draw per row from its temperature / top-k / top-p distribution (the
  * multinomial of src/generate.py:37 on explicit uniforms); greedy rows return the
  * first argmax (generate.py:24).  Row r uses Philox row row_base + r and `slot`.
- * workspace: lollm_sample_workspace_bytes(rows) bytes. */
+ * workspace: lollm_sample_workspace_bytes(rows) bytes: row statistics (152 bytes a row) and,
+ * for few rows, counts that let several workgroups share a long row; with room for the
+ * statistics alone every row takes one workgroup, with the same tokens. */
 long long lollm_sample_workspace_bytes(int rows);
 int lollm_sample_rows(const void* logits, int rows, int V, float inv_temperature, int top_k,
                       float top_p, uint64_t seed, uint64_t offset, const uint64_t* offset_dev,

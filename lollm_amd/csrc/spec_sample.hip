@@ -38,7 +38,9 @@
 //                bonus draw in two passes: ns workgroups per sequence sum the draw's
 //                weights over ns contiguous vocabulary slices, then one workgroup per
 //                sequence locates the slice holding the target and the token in it;
-//   sample_rows  one draw per row.
+//   sample_rows  one draw per row;
+//   sample_slices / sample_merge  statistics and draw of a few long rows, each spread over
+//                16 workgroups.
 // A draw is an inverse CDF over token ids in three steps: every wave of the block sums
 // the weights of its own contiguous sixteenth of the range (coalesced, exact integers,
 // the next 2-4 chunks per lane in flight), the sixteenth holding the target is summed
@@ -326,6 +328,23 @@ __device__ __forceinline__ void hist_chunk(uint4 u, uint32_t km2, int32_t dlim, 
   }
 }
 
+// The largest distance below the maximum key km that needs counting: all below SP_NBINS when
+// top-k reads the counts; without top-k only the mass (count x weight) is read, so distances
+// whose weight test t = (x - xmax) c >= -40 fails (weight 0) are skipped.  t does not increase
+// with the distance, so those distances are a suffix: bisect for its start over the distances
+// of real keys (skey >= -(0x7FFF - SP_MAG0)).
+__device__ __forceinline__ int32_t count_limit(int32_t km, float c, int top_k) {
+  if (top_k > 0) return SP_NBINS - 1;
+  const float xmax = key_value(km);
+  if (!((xmax - xmax) * c >= -40.0f)) return -1;   // the maximum is inf or NaN: every weight is zero
+  int lo = 0, hi = min(SP_NBINS - 1, km + (0x7FFF - SP_MAG0)) + 1;
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    if ((key_value(km - mid) - xmax) * c >= -40.0f) lo = mid; else hi = mid;
+  }
+  return lo;
+}
+
 // The rest of a sampled row's statistics once its maximum is known (top_bits: the bf16
 // bits of the largest logit): the distances that need counting, the per-key counts
 // (count(km2, dlim) fills hist; km2 = the maximum key mod 2^16 in both halves), then
@@ -346,24 +365,7 @@ __device__ __forceinline__ void row_stats_counts(uint32_t top_bits, float inv_te
   st.kmax = km;
   const float xmax = key_value(km);
   const float c = inv_temp * 1.44269504088896341f;
-  // ---- which distances need counting: all below SP_NBINS when top-k reads the counts;
-  //      without top-k only the mass (count x weight) is read, so distances whose weight
-  //      test t = (x - xmax) c >= -40 fails (weight 0) are skipped.  t does not increase
-  //      with the distance, so those distances are a suffix: bisect for its start over
-  //      the distances of real keys (skey >= -(0x7FFF - SP_MAG0)). ----
-  int32_t dlim = SP_NBINS - 1;
-  if (top_k <= 0) {
-    if (!((xmax - xmax) * c >= -40.0f)) {
-      dlim = -1;   // the maximum is inf or NaN: every weight is zero
-    } else {
-      int lo = 0, hi = min(SP_NBINS - 1, km + (0x7FFF - SP_MAG0)) + 1;
-      while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if ((key_value(km - mid) - xmax) * c >= -40.0f) lo = mid; else hi = mid;
-      }
-      dlim = lo;
-    }
-  }
+  const int32_t dlim = count_limit(km, c, top_k);
   // ---- per-key counts below the max ----
   const uint32_t km2 = ((uint32_t)km & 0xFFFFu) * 0x10001u;
   count(km2, dlim);
@@ -990,6 +992,217 @@ __global__ __launch_bounds__(SP_THREADS) void sample_rows_kernel(
   if (threadIdx.x == 0) out[r] = tok;
 }
 
+// Few rows: a row's statistics and draw spread over SP_SLICES workgroups.  A token's weight
+// depends only on its distance below the row's maximum, so the counts per distance of a slice
+// of the vocabulary give the slice's mass under any cut: the first kernel counts each slice
+// below the slice's own maximum, the second merges the counts (shifted to the row's maximum),
+// finds the cut, Z and the target as row_stats does, the slice that holds the target from the
+// slices' masses, and walks that slice alone.  Exact integers throughout: the same token as
+// row_stats + sample_rows, which read the row twice from one CU.
+// What bounds it: the chain of dependent loads, scans and barriers of the two kernels (one row
+// of 151936, top-k 20: 37.5 us on one CU, 21.3 here).
+constexpr int SP_SLICES = 16;
+constexpr int SP_SLICE_REG = 4;   // 16-byte chunks per thread held in registers
+struct SliceHead {
+  uint32_t top;    // the slice's maximum order key
+  int32_t n;       // distances 0 .. n - 1 are counted: every one that a cut can keep
+  uint32_t pad[2];
+};
+
+__device__ __forceinline__ void slice_range(int nch, int s, int& lo, int& hi) {
+  const int seg = (nch + SP_SLICES - 1) / SP_SLICES;
+  lo = min(s * seg, nch);
+  hi = min(lo + seg, nch);
+}
+
+__global__ __launch_bounds__(SP_THREADS) void sample_slices_kernel(
+    const uint16_t* __restrict__ logits, int V, float inv_temp, int top_k,
+    SliceHead* __restrict__ heads, uint16_t* __restrict__ counts) {
+  __shared__ uint32_t hist[SP_NBINS];
+  __shared__ uint64_t s64[16];
+  __shared__ int32_t last;
+  constexpr int PER = SP_NBINS / SP_THREADS;
+  const int tid = threadIdx.x;
+  const int slice = blockIdx.x, row = blockIdx.y;
+  const int nch = V >> 3;
+  int lo, hi;
+  slice_range(nch, slice, lo, hi);
+  const uint4* x4 = reinterpret_cast<const uint4*>(logits + (size_t)row * V);
+  uint4 reg[SP_SLICE_REG];
+#pragma unroll
+  for (int i = 0; i < SP_SLICE_REG; ++i) reg[i] = x4[min(lo + i * SP_THREADS + tid, nch - 1)];
+  for (int i = tid; i < SP_NBINS; i += SP_THREADS) hist[i] = 0u;
+  if (tid == 0) last = SP_NBINS;
+  uint32_t m2 = 0;
+#pragma unroll
+  for (int i = 0; i < SP_SLICE_REG; ++i)
+    if (lo + i * SP_THREADS + tid < hi) m2 = ord_max_chunk(m2, reg[i]);
+  for (int ch = lo + SP_SLICE_REG * SP_THREADS + tid; ch < hi; ch += SP_THREADS)
+    m2 = ord_max_chunk(m2, x4[ch]);
+  // (block_max's barriers also publish the zeroed counts)
+  const uint32_t top = (uint32_t)block_max<uint64_t>((uint64_t)max(m2 & 0xFFFFu, m2 >> 16), s64);
+  const int32_t km = skey(ord_bits(top));
+  // the slice's maximum is not above the row's, so a distance that weighs 0 below it weighs 0
+  // below the row's
+  const int32_t dlim = count_limit(km, inv_temp * 1.44269504088896341f, top_k);
+  const uint32_t km2 = ((uint32_t)km & 0xFFFFu) * 0x10001u;
+#pragma unroll
+  for (int i = 0; i < SP_SLICE_REG; ++i)
+    if (lo + i * SP_THREADS + tid < hi) hist_chunk(reg[i], km2, dlim, hist);
+  for (int ch = lo + SP_SLICE_REG * SP_THREADS + tid; ch < hi; ch += SP_THREADS)
+    hist_chunk(x4[ch], km2, dlim, hist);
+  __syncthreads();
+  uint32_t cnt[PER], csum = 0;
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    cnt[j] = hist[tid * PER + j];
+    csum += cnt[j];
+  }
+  if (top_k > 0) {   // the row's k-th largest is not below the slice's
+    uint32_t ctot;
+    const uint32_t cinc = block_inclusive_scan<uint32_t>(csum, reinterpret_cast<uint32_t*>(s64), &ctot);
+    const uint32_t c0 = cinc - csum;
+    if (c0 < (uint32_t)top_k && cinc >= (uint32_t)top_k) {
+      uint32_t run = c0;
+#pragma unroll
+      for (int j = 0; j < PER; ++j) {
+        run += cnt[j];
+        if (run >= (uint32_t)top_k) { last = tid * PER + j + 1; break; }
+      }
+    }
+    __syncthreads();
+  }
+  const int32_t n = lo < hi ? min(dlim + 1, last) : 0;
+  const size_t at = (size_t)row * SP_SLICES + slice;
+  static_assert(PER == 8, "one 16-byte store per thread");
+  if (tid * PER < n)
+    *reinterpret_cast<uint4*>(counts + at * SP_NBINS + tid * PER) =
+        make_uint4(cnt[0] | (cnt[1] << 16), cnt[2] | (cnt[3] << 16), cnt[4] | (cnt[5] << 16),
+                   cnt[6] | (cnt[7] << 16));
+  if (tid == 0) heads[at] = SliceHead{top, n, {0u, 0u}};
+}
+
+// The row's counts at distances d, d + SP_THREADS, .. (U of them) below its maximum; every load
+// is issued before the first is used (bins that a slice did not store are read and dropped).
+template <int U>
+__device__ __forceinline__ void merge_counts(const uint16_t* cr, const int32_t* n, const int32_t* shift,
+                                             int d, uint32_t* hist) {
+  uint16_t v[SP_SLICES][U];
+#pragma unroll
+  for (int s = 0; s < SP_SLICES; ++s)
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[s][u] = cr[s * SP_NBINS + max(d + u * SP_THREADS - shift[s], 0)];
+  uint32_t sum[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) sum[u] = 0u;
+#pragma unroll
+  for (int s = 0; s < SP_SLICES; ++s)
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int i = d + u * SP_THREADS - shift[s];
+      sum[u] += i >= 0 && i < n[s] ? (uint32_t)v[s][u] : 0u;
+    }
+#pragma unroll
+  for (int u = 0; u < U; ++u) hist[d + u * SP_THREADS] = sum[u];
+}
+
+// This lane's part of sum_{d < n} count[d] w[d], UN loads in flight.
+template <int UN>
+__device__ __forceinline__ uint64_t slice_mass(const uint32_t* cs, const uint64_t* w, int n) {
+  uint64_t acc = 0;
+  for (int p = threadIdx.x & 63; 2 * p < n; p += 64 * UN) {
+    uint32_t v[UN];
+#pragma unroll
+    for (int u = 0; u < UN; ++u) v[u] = cs[min(p + 64 * u, (n - 1) >> 1)];
+#pragma unroll
+    for (int u = 0; u < UN; ++u) {
+      const int d = 2 * (p + 64 * u);
+      if (d < n) acc += (uint64_t)(v[u] & 0xFFFFu) * w[d];
+      if (d + 1 < n) acc += (uint64_t)(v[u] >> 16) * w[d + 1];
+    }
+  }
+  return acc;
+}
+
+__global__ __launch_bounds__(SP_THREADS) void sample_merge_kernel(
+    const uint16_t* __restrict__ logits, int V, float inv_temp, int top_k, float top_p, uint64_t seed,
+    uint64_t offset_arg, const uint64_t* __restrict__ offset_dev, int row_base, int slot,
+    const SliceHead* __restrict__ heads, const uint16_t* __restrict__ counts, int32_t* __restrict__ out) {
+  __shared__ uint32_t hist[SP_NBINS];
+  __shared__ uint64_t tab[SP_NBINS];
+  __shared__ uint64_t s64[16], ms[SP_SLICES];
+  __shared__ int32_t shared_cut, found;
+  __shared__ uint64_t z_sh;
+  __shared__ RowStat sp_sh;
+  __shared__ int32_t n_sh[SP_SLICES], shift_sh[SP_SLICES];
+  __shared__ uint32_t top_sh;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int r = blockIdx.x;
+  const uint64_t offset = offset_dev ? *offset_dev : offset_arg;
+  const uint16_t* cr = counts + (size_t)r * SP_SLICES * SP_NBINS;
+  if (wave == 0) {
+    SliceHead hd = heads[(size_t)r * SP_SLICES + (lane & (SP_SLICES - 1))];
+    uint32_t top = hd.top;
+#pragma unroll
+    for (int m = 1; m < SP_SLICES; m <<= 1) top = max(top, (uint32_t)__shfl_xor((int)top, m, 64));
+    if (lane < SP_SLICES) {
+      n_sh[lane] = hd.n;
+      shift_sh[lane] = skey(ord_bits(top)) - skey(ord_bits(hd.top));
+    }
+    if (lane == 0) top_sh = top;
+  }
+  __syncthreads();
+  const float c = inv_temp * 1.44269504088896341f;
+  row_stats_counts(ord_bits(top_sh), inv_temp, top_k, top_p, &sp_sh, hist, s64, &shared_cut, &z_sh,
+                   [&](uint32_t, int32_t) {
+    int end = 0;
+#pragma unroll
+    for (int s = 0; s < SP_SLICES; ++s)
+      if (n_sh[s] > 0) end = max(end, n_sh[s] + shift_sh[s]);
+    for (int d0 = 0; d0 < SP_NBINS; d0 += 2 * SP_THREADS) {
+      if (end > d0 + SP_THREADS) {
+        merge_counts<2>(cr, n_sh, shift_sh, d0 + tid, hist);
+      } else {
+        if (end > d0) merge_counts<1>(cr, n_sh, shift_sh, d0 + tid, hist);
+        else hist[d0 + tid] = 0u;
+        hist[d0 + SP_THREADS + tid] = 0u;
+      }
+    }
+  });
+  __syncthreads();
+  const RowStat sp = sp_sh;
+  build_table(sp, c, tab);
+  __syncthreads();
+  // the slices' masses, a wave each
+  {
+    const int shift = shift_sh[wave], n = min(n_sh[wave], sp.cut + 1 - shift);
+    const uint32_t* cs = reinterpret_cast<const uint32_t*>(cr + wave * SP_NBINS);   // two counts
+    uint64_t acc = n <= 128 ? slice_mass<1>(cs, tab + shift, n) : slice_mass<16>(cs, tab + shift, n);
+    acc = wave_sum_any(acc);
+    if (lane == 0) ms[wave] = acc;
+  }
+  __syncthreads();
+  const uint32_t U = philox_u24(seed, offset, (uint32_t)(row_base + r), (uint32_t)slot);
+  const uint64_t tgt = (uint64_t)(((u128)U * sp.Z) >> 24);
+  uint64_t before = 0;
+  int slice = -1;
+  for (int s = 0; s < SP_SLICES; ++s) {
+    if (before + ms[s] > tgt) { slice = s; break; }
+    before += ms[s];
+  }
+  int32_t tok = V - 1;   // no mass: every weight is zero
+  if (slice >= 0) {
+    int lo, hi;
+    slice_range(V >> 3, slice, lo, hi);
+    const u32x4_t* v4 = reinterpret_cast<const u32x4_t*>(logits + (size_t)r * V);
+    auto ld = [=](int ch) { return v4[ch]; };
+    auto wt = [&](const u32x4_t& u, int ch, uint64_t* w) { chunk_weights(sp, tab, u, ch, w); };
+    draw_totals<uint64_t, SP_UN64>(lo, hi, ld, wt, s64);
+    tok = draw_refine<uint64_t>(lo, hi, ld, wt, s64, tgt - before, V, &found);
+  }
+  if (tid == 0) out[r] = tok;
+}
+
 // Repetition penalty (src/generate.py:18-22) in place on bf16 logit rows: a token of the
 // row's penalty set becomes bf16(x / p) if x > 0 else bf16(x * p), computed in fp32 as
 // torch computes bf16 arithmetic (one rounding of the fp32 quotient / product to bf16).
@@ -1144,9 +1357,26 @@ LOLLM_API long long lollm_spec_workspace_bytes(int B, int k, int with_draft) {
          (long long)B * accept_slices(B) * (SP_THREADS / 64) * (long long)sizeof(u128);
 }
 
+// Calls of few long rows, each slice countable in 16 bits, take the sliced kernels when the
+// workspace holds their counts.  These cost about the same whatever the row's length, and more
+// for more distances to merge: few with a top-k, up to SP_NBINS without (us, one workgroup per
+// row / sliced, 1 row and 16: top-k 20, V = 32000 21.0 / 20.9 and 21.8 / 21.4, 50304 24.1 / 21.0
+// and 25.1 / 22.8, 151936 37.5 / 21.3 and 38.7 / 24.3; T = 1.5 without top-k, 128256 34.5 / 33.6
+// and 35.5 / 36.9, 151936 38.6 / 33.4 and 39.9 / 37.1; 32 rows of 151936 40.8 / 42.9).
+constexpr int SP_SLICE_ROWS = 16;
+constexpr int SP_SLICE_FEW_K = 256;
+constexpr int SP_SLICE_MIN_V_FEW = 49152, SP_SLICE_MIN_V = 147456;
+constexpr int SP_SLICE_MAX_V = SP_SLICES * 65528;
+
+static long long slices_offset(long long rows) { return (stats_bytes(rows) + 15) / 16 * 16; }
+
+static long long slices_bytes(long long rows) {
+  return rows * SP_SLICES * (long long)(sizeof(SliceHead) + SP_NBINS * sizeof(uint16_t));
+}
+
 LOLLM_API long long lollm_sample_workspace_bytes(int rows) {
   if (rows <= 0) return -1;
-  return stats_bytes(rows);
+  return rows <= SP_SLICE_ROWS ? slices_offset(rows) + slices_bytes(rows) : stats_bytes(rows);
 }
 
 // lollm_spec_accept and lollm_spec_accept_rowmax: with target_rmax, the target rows'
@@ -1294,6 +1524,21 @@ LOLLM_API int lollm_sample_rows(const void* logits, int rows, int V, float inv_t
     if (rc) return rc;
     hipLaunchKernelGGL(argmax_final_kernel, dim3(rows), dim3(64), 0, st, (const uint64_t*)part,
                        (RowStat*)nullptr, out);
+    return launch_status();
+  }
+  const int min_v = top_k > 0 && top_k <= SP_SLICE_FEW_K ? SP_SLICE_MIN_V_FEW : SP_SLICE_MIN_V;
+  if (rows <= SP_SLICE_ROWS && V >= min_v && V <= SP_SLICE_MAX_V &&
+      (uintptr_t)workspace % 16 == 0 &&
+      workspace_bytes >= slices_offset(rows) + slices_bytes(rows)) {
+    SliceHead* heads = (SliceHead*)((char*)workspace + slices_offset(rows));
+    uint16_t* counts = (uint16_t*)(heads + (size_t)rows * SP_SLICES);
+    hipLaunchKernelGGL(sample_slices_kernel, dim3(SP_SLICES, rows), dim3(SP_THREADS), 0, st,
+                       (const uint16_t*)logits, V, inv_temperature, top_k, heads, counts);
+    int rc = launch_status();
+    if (rc) return rc;
+    hipLaunchKernelGGL(sample_merge_kernel, dim3(rows), dim3(SP_THREADS), 0, st,
+                       (const uint16_t*)logits, V, inv_temperature, top_k, top_p, seed, offset,
+                       offset_dev, row_base, slot, heads, counts, out);
     return launch_status();
   }
   int rc = launch_row_stats((const uint16_t*)logits, rows, nullptr, 0, V, inv_temperature, top_k,

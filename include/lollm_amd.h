@@ -79,7 +79,9 @@ int lollm_gdn_select_state(const float* snapshots, const int32_t* slot, float* s
  *   workspace  split-K partials, lollm_attn_workspace_bytes() bytes (required)
  *   grid     workgroups of the balanced split (0: one per CU of the current device,
  *            at most 1024): the 128-key blocks of all (sequence, KV head) pairs are
- *            dealt out to them in equal contiguous ranges
+ *            dealt out to them in equal contiguous ranges.  With 0, calls of 16 or more
+ *            queries a sequence with query tiles enough for the chip, or a short cache, run
+ *            one workgroup per (query tile, KV head) instead and leave the workspace alone
  *   scale    softmax scale (D^-0.5)
  * Supported: D == 256, Hq / Hkv <= 32, B <= 512. */
 long long lollm_attn_workspace_bytes(int B, int T, int Hq, int Hkv, int D, int max_len,
@@ -194,6 +196,13 @@ int lollm_verify_input(const int32_t* first, const int32_t* drafts, int k, const
 int lollm_mtp_input(const int32_t* tok, long long tok_stride, const void* hidden, long long ld_hidden,
                     const void* table, int vocab, const void* w_emb, const void* w_hidden, void* out,
                     int B, int H, float eps, void* stream);
+
+/* The same input of MTP.forward (mtp.py:61-73) from embedding rows: emb, hidden (B, L, H) bf16,
+ * out (B, L, 2H); and the block's vectors over an empty cache: lengths (B) = 0, kv_len (B) = L
+ * and rope (B, or NULL) = 1, the first of the positions 1..L.  Supported: H % 8 == 0, H <= 8192. */
+int lollm_mtp_rows(const void* emb, const void* hidden, const void* w_emb, const void* w_hidden,
+                   void* out, int B, int L, int H, float eps, int32_t* lengths, int32_t* kv_len,
+                   int32_t* rope, void* stream);
 
 /* SwiGLU of blocks.py:341-342 on a fused [gate | up] projection: gate_up (rows, 2F)
  * bf16 -> out (rows, F) = bf16(bf16(silu(gate)) * up).  Supported: F % 8 == 0. */

@@ -119,6 +119,35 @@ __global__ __launch_bounds__(RMS_THREADS) void mtp_input_kernel(const int32_t* _
   }
 }
 
+// The same input from embedding rows instead of ids (MTP.forward: src/qwen3_5/mtp.py:61-73), and
+// the block's position vectors: lengths[b] = 0, kv_len[b] = L and, where rope is given, rope[b]
+// = 1.  Every launch of the block waits for the one before it, about 4.5 us however little it
+// does; this one takes the place of two norms, a concatenation and three fills.
+__global__ __launch_bounds__(RMS_THREADS) void mtp_rows_kernel(const uint16_t* __restrict__ emb,
+                                                               const uint16_t* __restrict__ hidden,
+                                                               const uint16_t* __restrict__ w_emb,
+                                                               const uint16_t* __restrict__ w_hid,
+                                                               uint16_t* __restrict__ out, int H,
+                                                               float eps, int B, int L,
+                                                               int32_t* __restrict__ lengths,
+                                                               int32_t* __restrict__ kv_len,
+                                                               int32_t* __restrict__ rope) {
+  __shared__ float red[RMS_THREADS / 64];
+  const size_t row = blockIdx.x;
+  uint16_t* y = out + row * 2 * H;
+  if (blockIdx.y == 0) {
+    if (row == 0)
+      for (int b = threadIdx.x; b < B; b += RMS_THREADS) {
+        lengths[b] = 0;
+        kv_len[b] = L;
+        if (rope) rope[b] = 1;
+      }
+    rms_row(emb + row * H, nullptr, nullptr, w_emb, y, H, eps, red);
+  } else {
+    rms_row(hidden + row * H, nullptr, nullptr, w_hid, y + H, H, eps, red);
+  }
+}
+
 // The verify block's input: ids[b] = [first[b], drafts[b, 0 .. k)] (T = k + 1 tokens),
 // x[b, t] = table[ids[b, t]] (the embedding rows that open the residual stream) and
 // y[b, t] = RMSNorm_{1+w}(x[b, t]) (layer 0's input norm, the row arithmetic of
@@ -574,6 +603,18 @@ LOLLM_API int lollm_mtp_input(const int32_t* tok, long long tok_stride, const vo
   hipLaunchKernelGGL(mtp_input_kernel, dim3(B, 2), dim3(RMS_THREADS), 0, (hipStream_t)stream, tok,
                      tok_stride, (const uint16_t*)hidden, ld_hidden, (const uint16_t*)table, vocab,
                      (const uint16_t*)w_emb, (const uint16_t*)w_hidden, (uint16_t*)out, H, eps);
+  return launch_status();
+}
+
+LOLLM_API int lollm_mtp_rows(const void* emb, const void* hidden, const void* w_emb,
+                             const void* w_hidden, void* out, int B, int L, int H, float eps,
+                             int32_t* lengths, int32_t* kv_len, int32_t* rope, void* stream) {
+  if (!emb || !hidden || !w_emb || !w_hidden || !out || !lengths || !kv_len || B <= 0 || L <= 0 || H <= 0)
+    return LOLLM_EINVAL;
+  if (H % 8 || H > 8192 || (long long)B * L > 0x7FFFFFFF) return LOLLM_EUNSUPPORTED;
+  hipLaunchKernelGGL(mtp_rows_kernel, dim3(B * L, 2), dim3(RMS_THREADS), 0, (hipStream_t)stream,
+                     (const uint16_t*)emb, (const uint16_t*)hidden, (const uint16_t*)w_emb,
+                     (const uint16_t*)w_hidden, (uint16_t*)out, H, eps, B, L, lengths, kv_len, rope);
   return launch_status();
 }
 

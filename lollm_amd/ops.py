@@ -568,6 +568,24 @@ def mtp_input(tok, hidden, table, w_emb, w_hidden, eps, out=None):
     return out
 
 
+def mtp_rows(emb, hidden, w_emb, w_hidden, eps, rope=True):
+    """[RMSNorm_{1+w_emb}(emb) | RMSNorm_{1+w_hidden}(hidden)] (B, L, 2H) of (B, L, H) bf16 rows,
+    with the vectors of a block over an empty cache (lollm_mtp_rows): lengths 0, kv_len L and,
+    with rope, positions' first 1 (else None), (B,) int32 each."""
+    B, L, H = hidden.shape
+    _need(emb, "emb", torch.bfloat16, (B, L, H))
+    _need(hidden, "hidden", torch.bfloat16)
+    _need(w_emb, "w_emb", torch.bfloat16, (H,))
+    _need(w_hidden, "w_hidden", torch.bfloat16, (H,))
+    out = torch.empty(B, L, 2 * H, dtype=torch.bfloat16, device=hidden.device)
+    vec = torch.empty(3, -(-B // 4) * 4, dtype=torch.int32, device=hidden.device)[:, :B]
+    rc = _lib.lib().lollm_mtp_rows(
+        _ptr(emb), _ptr(hidden), _ptr(w_emb), _ptr(w_hidden), _ptr(out), B, L, H, float(eps),
+        _ptr(vec[0]), _ptr(vec[1]), _ptr(vec[2]) if rope else None, _stream())
+    _lib.check(rc, "lollm_mtp_rows")
+    return out, vec[0], vec[1], vec[2] if rope else None
+
+
 def verify_input(first, drafts, table, w, eps, lengths=None, *, ids=None, x=None, y=None,
                  kv_len=None):
     """The verify block's input in one kernel (lollm_verify_input): ids = [first | drafts]
@@ -709,7 +727,7 @@ def gdn_chunked_ok(T, slots, win_rows, conv_kernel, proj_stride=0):
 
 # Heads of a call (B * Hv) up to which its chunks, when there are several, are spread over the
 # chip; more heads fill it walking their own chunks (us, spread / walked, 32 heads a sequence:
-# 1 x 1847 tokens 146 / 543, 3 x 1500 274 / 453, 4 x 1000 229 / 308, 5 x 1638 515 / 499,
+# 1 x 1847 tokens 130 / 543, 3 x 1500 274 / 453, 4 x 1000 229 / 308, 5 x 1638 515 / 499,
 # 8 x 1024 461 / 320; 1 x 100 32 / 46, 1 x 64 28 / 28).
 GDN_SPLIT_MAX_HEADS = 128
 GDN_CHUNK = 64

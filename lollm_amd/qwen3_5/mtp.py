@@ -49,16 +49,18 @@ class MTP:
                                [self.fc] + layer.self_attn.projections() + layer.mlp.projections()),
                            model.device)
 
-    def _block(self, hidden, next_emb, k_cache, v_cache, lengths, kv_len, rope_pos, ws, tok=None):
+    def _block(self, hidden, next_emb, k_cache, v_cache, lengths, kv_len, rope_pos, ws, tok=None,
+               fc_in=None):
         """Returns (MTP layer output before the final norm, normed output).  Given the
         next tokens' ids `tok` (B,) int32 instead of their embeddings, the lookup, both
-        pre-fc norms and the concatenation run as one kernel (lollm_mtp_input)."""
-        if tok is not None:
+        pre-fc norms and the concatenation run as one kernel (lollm_mtp_input); fc_in: that
+        input, formed already."""
+        if fc_in is None and tok is not None:
             B = tok.numel()
             fc_in = ops.mtp_input(tok, hidden, self.model.model.embed_tokens.weight,
                                   self.pre_fc_norm_embedding.weight, self.pre_fc_norm_hidden.weight,
                                   self.pre_fc_norm_embedding.eps).view(B, 1, -1)
-        else:
+        elif fc_in is None:
             fc_in = torch.cat([self.pre_fc_norm_embedding(next_emb),
                                self.pre_fc_norm_hidden(hidden)], -1)
         layer = self.layers[0]
@@ -81,9 +83,13 @@ class MTP:
         """mtp.py:61-73: (B, L, H) -> normalised MTP hidden (B, L, H)."""
         B, L, _ = hidden.shape
         dev = self.model.device
-        if positions is None:
-            rope = torch.ones(B, dtype=torch.int32, device=dev)        # positions 1..L
-        else:
+        hidden = hidden.to(torch.bfloat16).contiguous()
+        next_emb = next_emb.to(torch.bfloat16).contiguous()
+        e, h = self.pre_fc_norm_embedding, self.pre_fc_norm_hidden
+        # default positions: 1..L
+        fc_in, zeros, kv_len, rope = ops.mtp_rows(next_emb, hidden, e.weight, h.weight, e.eps,
+                                                  rope=positions is None)
+        if positions is not None:
             # any positions vector (L,) shared by the batch, as mtp.py:64-67, or (B, L)
             pos = torch.as_tensor(positions, device=dev).to(torch.int32)
             if pos.dim() == 1:
@@ -91,12 +97,11 @@ class MTP:
             if tuple(pos.shape) != (B, L):
                 raise ValueError(f"positions must be ({L},) or ({B}, {L}), got {tuple(positions.shape)}")
             rope = pos.contiguous()
-        kc, vc = self.scratch_cache(B, L)
-        zeros = torch.zeros(B, dtype=torch.int32, device=dev)
-        kv_len = torch.full((B,), L, dtype=torch.int32, device=dev)
-        _, normed = self._block(hidden.to(torch.bfloat16).contiguous(),
-                                next_emb.to(torch.bfloat16).contiguous(), kc, vc, zeros, kv_len,
-                                rope, None)
+        # every cache row is written before it is read
+        shape = (B, self.cfg.num_key_value_heads, L, self.cfg.head_dim)
+        kc = torch.empty(shape, dtype=torch.bfloat16, device=dev)
+        vc = torch.empty(shape, dtype=torch.bfloat16, device=dev)
+        _, normed = self._block(hidden, next_emb, kc, vc, zeros, kv_len, rope, None, fc_in=fc_in)
         return normed
 
     __call__ = forward

@@ -148,8 +148,8 @@ def marker():
 def projection_paths(model, mtp, B, k):
     """The path of each projection shape of the step ("gemm grid g, c-col groups" =
     lollm_gemm on g workgroups with c-column groups -- 96 where those divide over the
-    grid and 64-column ones would not, the library's rule -- "blas" = hipBLASLt; a fixed
-    function of the shape), keyed "NxK M=rows"."""
+    grid and 64-column ones would not, the library's rule -- "blas" = lollm_gemm_rows or
+    hipBLASLt; a fixed function of the shape), keyed "NxK M=rows"."""
     out = {}
     layers = list(model.model.layers) + list(mtp.layers)
     projs = [model.lm_head, mtp.fc]

@@ -1,5 +1,5 @@
-"""The many-row GEMM (lollm_gemm_rows) against fp32, at the edges of its tiles, and its row
-independence of M and tile; the rule that picks its tile is checked on the CPU."""
+"""The many-row GEMM (lollm_gemm_rows) against fp32, at the edges of its tiles, and, with K
+whole, its row independence of M and tile; the rule that picks its tile is checked on the CPU."""
 
 import pytest
 import torch

@@ -708,13 +708,11 @@ def attn_small(qkv, q_norm_w, k_norm_w, inv_freq, lengths, kv_len, B, Hq, Hkv, D
     return out
 
 
-# Long calls that take the chunked form: a chunk costs a workgroup about the same time whatever
-# it holds, the recurrence 2.2 us per token and round of heads (us, chunked / recurrent, 32
-# heads a sequence: 24 tokens x 1 sequence 27 / 58, x 64 255 / 316; 12 tokens x 8 34 / 45, x 32
-# 127 / 106; 63 tokens x 1 28 / 141).
-GDN_CHUNK_MIN_T = 24
-GDN_CHUNK_MIN_T_FEW = 12
-GDN_CHUNK_FEW_HEADS = 256
+# Long calls from this many tokens on take the chunked form: a whole chunk.  Shorter ones keep the
+# recurrence although a chunk would be faster (us, chunked / recurrent, 32 heads: 63 tokens x 1
+# sequence 28 / 141, 24 x 64 255 / 316): its products are fp32 where the chunk's fp32 operands
+# enter with 16 bits, and its softplus keeps the small gates that the chunk's logarithm rounds off.
+GDN_CHUNK_MIN_T = 64
 
 
 def gdn_chunked_ok(T, slots, win_rows, conv_kernel, proj_stride=0):
@@ -756,8 +754,7 @@ def gdn_layer(proj, conv_w, A_log, dt_bias, norm_w, win, conv_off, rec, rec_half
     conv_dim) bf16; rec (B, 2, Hv, D, D) fp32 state halves; rep (B, 2, Hv, S,
     gdn_record_bytes(D)) uint8 replay records; conv_off / rec_half / replay (B,) int32.
     chunked: None = the chunked kernels for long calls of at least GDN_CHUNK_MIN_T tokens
-    (GDN_CHUNK_MIN_T_FEW with few heads) that they support, the recurrent kernel otherwise;
-    True / False force one."""
+    that they support, the recurrent kernel otherwise; True / False force one."""
     P = proj.shape[-1]
     _need(proj, "proj", torch.bfloat16)
     _need(win, "win", torch.bfloat16)
@@ -770,8 +767,7 @@ def gdn_layer(proj, conv_w, A_log, dt_bias, norm_w, win, conv_off, rec, rec_half
         out = torch.empty(B, T, value_dim, dtype=torch.bfloat16, device=proj.device)
     W = win.shape[1] // 2
     if chunked is None:
-        chunked = (T >= (GDN_CHUNK_MIN_T_FEW if B * Hv <= GDN_CHUNK_FEW_HEADS else GDN_CHUNK_MIN_T)
-                   and gdn_chunked_ok(T, S, W, conv_kernel, P))
+        chunked = T >= GDN_CHUNK_MIN_T and gdn_chunked_ok(T, S, W, conv_kernel, P)
     fn, ws = "lollm_gdn_layer_chunked" if chunked else "lollm_gdn_layer", ()
     if chunked and T > GDN_CHUNK and B * Hv <= GDN_SPLIT_MAX_HEADS:
         need = _lib.lib().lollm_gdn_split_workspace_bytes(B, T, Hk, Hv)

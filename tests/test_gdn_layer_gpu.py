@@ -288,6 +288,17 @@ def test_gdn_layer_chunked_agrees_with_recurrent():
         torch.testing.assert_close(rc[b, o], rr[b, o], rtol=2e-2, atol=2e-2 * scale)
 
 
+@pytest.mark.parametrize("B,T", [(1, 9), (2, 13), (9, 24), (1, 40), (1, 63)])
+def test_gdn_layer_below_a_chunk_is_the_recurrence(B, T):
+    """A long call of fewer tokens than a chunk computes in fp32 throughout: outputs and
+    states are the recurrent kernel's bit for bit, whatever the batch."""
+    print(f"case gdn_layer below a chunk B={B} T={T}", flush=True)
+    m = make(B, T, 4, T)
+    got, dev = run(m, m["proj"])
+    ref, dev0 = run(m, m["proj"], chunked=False)
+    assert torch.equal(got, ref) and torch.equal(dev["rec"].cpu(), dev0["rec"].cpu())
+
+
 @pytest.mark.parametrize("B,T,S,seed", [(2, 2048, 4, 7), (1, 4100, 8, 11)])
 def test_gdn_layer_chunked_precision_long(B, T, S, seed):
     """Over 32-65 chunks the chunked kernel (bf16 MFMA products with hi/lo operand

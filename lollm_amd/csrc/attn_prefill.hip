@@ -13,6 +13,13 @@
 // per block) and are read by all four waves; wave w owns rows 32 RG w .. of the tile with
 // its Q in registers and its O^T in accumulator registers.
 //
+// Precision.  One running maximum serves a row where the split-K kernels have one per wave and
+// piece, whose largest weights are 1 and lose nothing as bf16; so weights enter the product with
+// V as hi + lo bf16 (16 bits) and the row sum as they are, fp32.  Relative error against 64 bits
+// (2 x 1999 tokens, normal q, k, v): split-K 2.07e-3, weights in bf16 here 2.12e-3, hi + lo
+// 1.66e-3, which is the output's own rounding to bf16.  It costs a third of the products: 185 ->
+// 221 us.
+//
 // What bounds it: operand reads and the softmax beside the products.  A 32x32x16 MFMA
 // (32 cycles) takes a 1 KB operand from LDS, and the four waves of a CU then need 128 B per
 // cycle, the LDS peak.  With RG = 2 a wave reuses each K / V operand for two row groups and
@@ -20,9 +27,9 @@
 // registers, Q half of the vector registers.  A lone wave overlaps nothing by itself, so the
 // exponentials of block j + 1 are placed between the products of V with block j.
 //
-// Measured (us, causal, T = kv length, split-K kernels before / RG = 1 / RG = 2): 2 x 1999,
-// 32 q / 4 kv heads 1048 / 223 / 195 (673 TFLOP/s); 1 x 4096 1830 / 341 / 299 (919 TFLOP/s);
-// 3 x 1500 1120 / 189 / 186; 32 x 128 over 1128 keys 912 / 235 / 215.
+// Measured (us, causal, T = kv length, split-K kernels / RG = 1 / RG = 2): 2 x 1999,
+// 32 q / 4 kv heads 1020 / 247 / 222 (591 TFLOP/s); 1 x 4096 1822 / 407 / 372 (740 TFLOP/s);
+// 3 x 1500 1110 / 216 / 217; 32 x 128 over 1128 keys 903 / 260 / 244.
 //
 // Rows of K and V are 512 bytes in LDS with no padding (the DMA writes 1 KB runs); the
 // 16-byte chunk c of row r sits at c ^ (r & 15) for K and c ^ (2 (r & 7)) for V, so the
@@ -35,7 +42,7 @@ namespace lollm {
 constexpr int AP_WAVES = 4;
 constexpr int AP_MIN_T = 16;
 constexpr int AP_KEYS = 32;                    // keys per block
-constexpr int AP_AHEAD = 4;                    // operands read ahead of their products
+constexpr int AP_AHEAD = 3;                    // operands read ahead of their products
 constexpr int AP_SET = AP_KEYS * AT_D * 2;     // 16 KB: K or V rows of a block
 
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -66,12 +73,12 @@ __device__ __forceinline__ void ap_mfma(f32x16& s, bf16x8 k, bf16x8 q) {
 // the wait states between the last product and the first VALU access of its result
 __device__ __forceinline__ void ap_mfma_done(f32x16& s) { asm volatile("s_nop 15\n\ts_nop 7" : "+v"(s)); }
 
-// s + both of a pair of rounded weights.  The row sum is taken over the weights as the product
-// with V sees them (bf16), so a row that few keys dominate is normalised exactly: the error
-// against 64 bits is smaller than with the sum of the unrounded weights.
-__device__ __forceinline__ float ap_add2(bf16x2 p, float s) {
-  const bf16x2 one = {(__bf16)1.f, (__bf16)1.f};
-  return __builtin_amdgcn_fdot2_f32_bf16(p, one, s, false);
+// A pair of fp32 weights as bf16 hi and lo, x = hi + lo to 16 bits.
+__device__ __forceinline__ void ap_split(float x, float y, uint32_t& hi, uint32_t& lo) {
+  const bf16x2 h = {(__bf16)x, (__bf16)y};
+  hi = __builtin_bit_cast(uint32_t, h);
+  const bf16x2 l = {(__bf16)(x - __uint_as_float(hi << 16)), (__bf16)(y - __uint_as_float(hi & 0xffff0000u))};
+  lo = __builtin_bit_cast(uint32_t, l);
 }
 __device__ __forceinline__ int ap_div(int r, uint32_t mul) { return (int)(((uint32_t)r * mul) >> 16); }
 
@@ -171,7 +178,7 @@ __global__ __launch_bounds__(64 * AP_WAVES, 1) void attn_prefill_kernel(ApArgs a
 
   f32x16 O[RG][8];   // O^T: 32 columns x 32 rows per tile; lane's row = l32
   float m_ref[RG], l_s[RG];
-  bf16x8 P[RG][2];   // exp of the block whose V comes next
+  bf16x8 P[RG][2], Pl[RG][2];   // exp of the block whose V comes next, hi and lo
 #pragma unroll
   for (int rg = 0; rg < RG; ++rg) {
     m_ref[rg] = -INFINITY;
@@ -271,7 +278,7 @@ __global__ __launch_bounds__(64 * AP_WAVES, 1) void attn_prefill_kernel(ApArgs a
       return __builtin_bit_cast(bf16x8, u32x4_t{w0.x, w0.y, w1.x, w1.y});
     };
     bf16x8 vf[AP_AHEAD];
-    u32x4_t Pn[RG][2];
+    u32x4_t Pn[RG][2], Pm[RG][2];
     float pe[RG];
 #pragma unroll
     for (int i = 0; i < AP_AHEAD; ++i) vf[i] = read_v(i);
@@ -280,16 +287,20 @@ __global__ __launch_bounds__(64 * AP_WAVES, 1) void attn_prefill_kernel(ApArgs a
 #pragma unroll
       for (int rg = 0; rg < RG; ++rg)
         O[rg][n >> 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[n % AP_AHEAD], P[rg][n & 1], O[rg][n >> 1], 0, 0, 0);
+#pragma unroll
+      for (int rg = 0; rg < RG; ++rg)
+        O[rg][n >> 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[n % AP_AHEAD], Pl[rg][n & 1], O[rg][n >> 1], 0, 0, 0);
       if (n + AP_AHEAD < 16) vf[n % AP_AHEAD] = read_v(n + AP_AHEAD);
 #pragma unroll
       for (int rg = 0; rg < RG; ++rg) {
         const float p = fast_exp2(__builtin_fmaf(S[rg][n], a.cl2, -base[rg]));
         if (n & 1) {   // (pinned here: the compiler would sink them all past the rescale)
-          const bf16x2 t = {(__bf16)pe[rg], (__bf16)p};
-          l_s[rg] = ap_add2(t, l_s[rg]);
-          uint32_t w = __builtin_bit_cast(uint32_t, t);
-          asm volatile("" : "+v"(w), "+v"(l_s[rg]));
-          Pn[rg][n >> 3][(n & 7) >> 1] = w;
+          uint32_t hi, lo;
+          ap_split(pe[rg], p, hi, lo);
+          l_s[rg] += pe[rg] + p;
+          asm volatile("" : "+v"(hi), "+v"(lo), "+v"(l_s[rg]));
+          Pn[rg][n >> 3][(n & 7) >> 1] = hi;
+          Pm[rg][n >> 3][(n & 7) >> 1] = lo;
         } else {
           pe[rg] = p;
         }
@@ -297,10 +308,12 @@ __global__ __launch_bounds__(64 * AP_WAVES, 1) void attn_prefill_kernel(ApArgs a
       __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
-    for (int rg = 0; rg < RG; ++rg) {
-      P[rg][0] = __builtin_bit_cast(bf16x8, Pn[rg][0]);
-      P[rg][1] = __builtin_bit_cast(bf16x8, Pn[rg][1]);
-    }
+    for (int rg = 0; rg < RG; ++rg)
+#pragma unroll
+      for (int k2 = 0; k2 < 2; ++k2) {
+        P[rg][k2] = __builtin_bit_cast(bf16x8, Pn[rg][k2]);
+        Pl[rg][k2] = __builtin_bit_cast(bf16x8, Pm[rg][k2]);
+      }
     rescale();
   };
 
@@ -309,13 +322,21 @@ __global__ __launch_bounds__(64 * AP_WAVES, 1) void attn_prefill_kernel(ApArgs a
     scores(ks0, 0);
 #pragma unroll
     for (int rg = 0; rg < RG; ++rg) {
+      u32x4_t Pn[2], Pm[2];
 #pragma unroll
       for (int r = 0; r < 16; r += 2) {
-        const bf16x2 t = {(__bf16)fast_exp2(__builtin_fmaf(S[rg][r], a.cl2, -base[rg])),
-                          (__bf16)fast_exp2(__builtin_fmaf(S[rg][r + 1], a.cl2, -base[rg]))};
-        l_s[rg] = ap_add2(t, l_s[rg]);
-        P[rg][r >> 3][r & 7] = t[0];
-        P[rg][r >> 3][(r & 7) + 1] = t[1];
+        const float p0 = fast_exp2(__builtin_fmaf(S[rg][r], a.cl2, -base[rg]));
+        const float p1 = fast_exp2(__builtin_fmaf(S[rg][r + 1], a.cl2, -base[rg]));
+        uint32_t hi, lo;
+        ap_split(p0, p1, hi, lo);
+        l_s[rg] += p0 + p1;
+        Pn[r >> 3][(r & 7) >> 1] = hi;
+        Pm[r >> 3][(r & 7) >> 1] = lo;
+      }
+#pragma unroll
+      for (int k2 = 0; k2 < 2; ++k2) {
+        P[rg][k2] = __builtin_bit_cast(bf16x8, Pn[k2]);
+        Pl[rg][k2] = __builtin_bit_cast(bf16x8, Pm[k2]);
       }
     }
     rescale();
@@ -406,15 +427,15 @@ int attn_prefill_groups(int B, int T, int Hkv, int n_rep, int max_len, int cus) 
   // Verify-sized calls keep the split-K kernels, whose rows do not depend on T.
   if (T < AP_MIN_T) return 0;
   const long long rows = (long long)T * n_rep, pairs = (long long)B * Hkv;
-  // 256-row tiles cost 1.65 of a 128-row tile's time; worth it once two rounds of them fill
-  // the chip (448 tiles of 1500 keys: equal; 512 of 2000 - 4096: 12 - 14% faster; 128 tiles of
-  // 8256 keys 413 us against 264)
-  if (4 * pairs * ((rows + 255) / 256) >= 7LL * cus) return 2;
-  // A lone tile walks its keys at 0.03 us each; the split kernels take 0.0004 us per key and
-  // tile: from 64 tiles on this kernel is faster (64 tiles of 1024 keys 44 us against 54,
-  // 28 of 4000 130 against 78), and below 512 keys its single launch is (36 tiles of 200
-  // keys: 22 against 31)
-  if (4 * pairs * ((rows + 127) / 128) >= cus || max_len <= 512) return 1;
+  // 256-row tiles cost 1.7 of a 128-row tile's time; worth it from one and a half rounds of them
+  // (us, RG = 1 / 2: 384 tiles of 3072 keys 256 / 242, 400 of 1600 161 / 150, 512 of 4096 407 /
+  // 372; 128 tiles of 8256 keys 368 / 521)
+  if (2 * pairs * ((rows + 255) / 256) >= 3LL * cus) return 2;
+  // A lone tile walks its keys at 0.038 us each; the split kernels take 0.00048 us per key and
+  // tile: from 80 tiles on this kernel is the faster one whatever the length (us, long / split:
+  // 128 tiles of 500 keys 33 / 75; 64 of 1024 51 / 54, of 2000 84 / 83, of 4000 153 / 124; 56
+  // of 4000 153 / 110), and below 512 keys its single launch is (52 tiles of 200 keys: 22 / 37)
+  if (16 * pairs * ((rows + 127) / 128) >= 5LL * cus || max_len <= 512) return 1;
   return 0;
 }
 

@@ -79,9 +79,11 @@ int lollm_gdn_select_state(const float* snapshots, const int32_t* slot, float* s
  *   workspace  split-K partials, lollm_attn_workspace_bytes() bytes (required)
  *   grid     workgroups of the balanced split (0: one per CU of the current device,
  *            at most 1024): the 128-key blocks of all (sequence, KV head) pairs are
- *            dealt out to them in equal contiguous ranges.  With 0, calls of 16 or more
- *            queries a sequence with query tiles enough for the chip, or a short cache, run
- *            one workgroup per (query tile, KV head) instead and leave the workspace alone
+ *            dealt out to them in equal contiguous ranges.  With 0, calls of more than 64
+ *            tokens in all and 16 or more a sequence, with query tiles enough for the chip,
+ *            run one workgroup per (query tile, KV head) instead and leave the workspace
+ *            alone; a verify call of that size passes the grid, and a row's bits then do not
+ *            depend on T
  *   scale    softmax scale (D^-0.5)
  * Supported: D == 256, Hq / Hkv <= 32, B <= 512. */
 long long lollm_attn_workspace_bytes(int B, int T, int Hq, int Hkv, int D, int max_len,

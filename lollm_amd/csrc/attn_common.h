@@ -35,7 +35,7 @@ __device__ __forceinline__ float sigmoidf_(float x) { return 1.f / (1.f + __expf
 
 // Row groups per wave of the long-call kernel (attn_prefill.hip) for this geometry on a device
 // with `cus` CUs, or 0 where the split-K kernels are the faster ones.
-int attn_prefill_groups(int B, int T, int Hkv, int n_rep, int max_len, int cus);
+int attn_prefill_groups(int B, int T, int Hkv, int n_rep, int cus);
 int attn_prefill_launch(const AttnArgs& a, int groups, hipStream_t st);
 
 }  // namespace lollm

@@ -40,7 +40,8 @@
 namespace lollm {
 
 constexpr int AP_WAVES = 4;
-constexpr int AP_MIN_T = 16;
+constexpr int AP_MIN_T = 16;                   // new positions per sequence
+constexpr int AP_FEW_ROWS = 64;                // tokens of a call that keeps the split-K kernels
 constexpr int AP_KEYS = 32;                    // keys per block
 constexpr int AP_AHEAD = 3;                    // operands read ahead of their products
 constexpr int AP_SET = AP_KEYS * AT_D * 2;     // 16 KB: K or V rows of a block
@@ -423,9 +424,11 @@ __global__ __launch_bounds__(64 * AP_WAVES, 1) void attn_prefill_kernel(ApArgs a
   }
 }
 
-int attn_prefill_groups(int B, int T, int Hkv, int n_rep, int max_len, int cus) {
-  // Verify-sized calls keep the split-K kernels, whose rows do not depend on T.
-  if (T < AP_MIN_T) return 0;
+int attn_prefill_groups(int B, int T, int Hkv, int n_rep, int cus) {
+  // A sequence's numbers do not depend on how its tokens are divided into calls of up to 64 (the
+  // few-row GEMMs' limit): those keep the split-K kernels, whose rows do not depend on T.  Nor do
+  // they depend on the cache's capacity, so the lines below go by the queries alone.
+  if (T < AP_MIN_T || (long long)B * T <= AP_FEW_ROWS) return 0;
   const long long rows = (long long)T * n_rep, pairs = (long long)B * Hkv;
   // 256-row tiles cost 1.7 of a 128-row tile's time; worth it from one and a half rounds of them
   // (us, RG = 1 / 2: 384 tiles of 3072 keys 256 / 242, 400 of 1600 161 / 150, 512 of 4096 407 /
@@ -434,8 +437,8 @@ int attn_prefill_groups(int B, int T, int Hkv, int n_rep, int max_len, int cus) 
   // A lone tile walks its keys at 0.038 us each; the split kernels take 0.00048 us per key and
   // tile: from 80 tiles on this kernel is the faster one whatever the length (us, long / split:
   // 128 tiles of 500 keys 33 / 75; 64 of 1024 51 / 54, of 2000 84 / 83, of 4000 153 / 124; 56
-  // of 4000 153 / 110), and below 512 keys its single launch is (52 tiles of 200 keys: 22 / 37)
-  if (16 * pairs * ((rows + 127) / 128) >= 5LL * cus || max_len <= 512) return 1;
+  // of 4000 153 / 110)
+  if (16 * pairs * ((rows + 127) / 128) >= 5LL * cus) return 1;
   return 0;
 }
 

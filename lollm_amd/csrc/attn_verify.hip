@@ -571,7 +571,7 @@ LOLLM_API int lollm_attn_verify(const void* q, const void* k_cache, const void* 
   a.cl2 = scale * 1.4426950408889634f;
   hipStream_t st = (hipStream_t)stream;
   if (grid == 0) {
-    const int groups = attn_prefill_groups(B, T, Hkv, n_rep, max_len, nw);
+    const int groups = attn_prefill_groups(B, T, Hkv, n_rep, nw);
     if (groups) return attn_prefill_launch(a, groups, st);
   }
   hipLaunchKernelGGL(attn_verify_kernel, dim3(nw), dim3(AW_THREADS), 0, st, a);

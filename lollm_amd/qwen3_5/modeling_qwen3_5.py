@@ -17,7 +17,7 @@ import torch
 import torch.nn.functional as F
 
 from .. import ops
-from .blocks import MLP, GatedAttention, GatedDeltaNet, Projection, RMSNorm, rope_inv_freq
+from .blocks import MLP, GatedAttention, GatedDeltaNet, Projection, RMSNorm, _cus, rope_inv_freq
 from .config import Qwen3_5Config
 from .kv import Qwen3_5Cache
 
@@ -125,6 +125,9 @@ class Qwen3_5Model:
         else:
             x, h_first, kv_len = inputs
         ws = self.attn_workspace(B, T, cache.max_len)
+        # a call that can be rolled back (the verify block, as the GDN layers tell it) asks for
+        # the split-K attention at any size, where a row's bits do not depend on T
+        grid = self.attn_grid or (_cus() if T <= cache.spec_slots else 0)
         # each residual-stream projection (o_proj / out_proj / down_proj) is issued with
         # the residual add and the norm that follows it (modeling_qwen3_5.py:59-60)
         pending = None   # (down_proj, its input): opens the next layer
@@ -137,7 +140,7 @@ class Qwen3_5Model:
                 s = cache.layers[i]
                 mixer = layer.self_attn
                 core = mixer.core(h_in, s["k"], s["v"], lengths, kv_len,
-                                  grid=self.attn_grid, workspace=ws)
+                                  grid=grid, workspace=ws)
             else:
                 mixer = layer.linear_attn
                 core = mixer.core(h_in, cache, i)

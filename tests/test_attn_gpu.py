@@ -119,6 +119,35 @@ def test_attn_rows_do_not_depend_on_T(Hq, Hkv, base, grid):
         assert torch.equal(part.cpu(), full[:, :t].cpu()), t
 
 
+@pytest.mark.parametrize("B,T,Hq,Hkv,base", [(1, 20, 32, 4, 130), (2, 17, 8, 2, 130), (4, 16, 32, 4, 130),
+                                             (1, 64, 32, 4, 130), (1, 64, 256, 8, 60)])
+def test_attn_rows_do_not_depend_on_T_up_to_64_tokens(B, T, Hq, Hkv, base):
+    """The same for calls of up to 64 tokens in all, also with tiles enough for the long-call
+    kernel (8 KV heads of 32 query heads: 128) and over a short cache.  Every key block has a
+    workgroup of its own, and at most two a sequence, whose sum has one order only."""
+    from lollm_amd import ops
+    print(f"case attn rows B={B} T={T} Hq={Hq} Hkv={Hkv}", flush=True)
+    base = [base + 9 * b for b in range(B)]
+    q, kc, vc, kl, gate = make_case(B, T, Hq, Hkv, [b + T for b in base], seed=T + Hq)
+    full = ops.attn_verify(q.cuda(), kc.cuda(), vc.cuda(), kl.cuda(), gate.cuda())
+    for t in (1, 4, T - 1):
+        part = ops.attn_verify(q[:, :t].contiguous().cuda(), kc.cuda(), vc.cuda(),
+                               (kl - (T - t)).cuda(), gate[:, :t].contiguous().cuda())
+        assert torch.equal(part.cpu(), full[:, :t].cpu()), t
+
+
+@pytest.mark.parametrize("B,T,Hq,Hkv,L", [(1, 200, 32, 4, 200), (2, 40, 8, 2, 300), (4, 200, 32, 4, 333)])
+def test_attn_does_not_depend_on_the_cache_capacity(B, T, Hq, Hkv, L):
+    """The same call over caches of different capacity gives the same bits, on either side of
+    the long-call kernel's line."""
+    from lollm_amd import ops
+    print(f"case attn capacity B={B} T={T} Hq={Hq} Hkv={Hkv} L={L}", flush=True)
+    q, kc, vc, kl, gate = make_case(B, T, Hq, Hkv, [L] * B, seed=T + L, max_len=900)
+    outs = [ops.attn_verify(q.cuda(), kc[:, :, :n].contiguous().cuda(), vc[:, :, :n].contiguous().cuda(),
+                            kl.cuda(), gate.cuda()).cpu() for n in (L, 900)]
+    assert torch.equal(*outs)
+
+
 def test_attn_workspace_is_validated():
     """A workspace smaller than lollm_attn_workspace_bytes is refused, not overrun."""
     from lollm_amd import ops

@@ -98,6 +98,38 @@ def test_rollback_equals_shorter_history(micro):
         close_logits(lg[b, -1], ref[0, -1], r16[0, -1])
 
 
+def test_long_verify_block_equals_short_one(micro):
+    """A verify block of 1 + k = 20 tokens (k = 19) gives its first rows the bits of a block of
+    5 and of 16, as a rollback to a short accepted prefix needs: 40 rows, so every GEMM is the
+    few-row one, and within one key block of the attention."""
+    model, _, _, cfg = micro
+    print("case long verify block", flush=True)
+    g = torch.Generator().manual_seed(6)
+    prompt = torch.randint(0, cfg.vocab_size, (2, 70), generator=g).cuda()
+    blk = torch.randint(0, cfg.vocab_size, (2, 20), generator=g).cuda()
+    hidden = []
+    for t in (20, 5, 16):
+        cache = model.new_cache(2, 120, spec_slots=20)
+        model(prompt, cache)
+        hidden.append(model.hidden_states(blk[:, :t].contiguous(), cache)[0])
+    for h in hidden[1:]:
+        assert torch.equal(h, hidden[0][:, :h.shape[1]])
+
+
+def test_verify_block_asks_for_the_split_attention(micro, monkeypatch):
+    """A block within the cache's slots keeps the split-K attention past 64 rows too; a prompt
+    of the same size leaves the choice to the library."""
+    from lollm_amd import ops
+    model, _, _, cfg = micro
+    grids, plain = [], ops.attn_verify
+    monkeypatch.setattr(ops, "attn_verify", lambda *a, grid=0, **kw: grids.append(grid) or plain(*a, grid=grid, **kw))
+    ids = torch.zeros(8, 16, dtype=torch.long, device="cuda")
+    for slots in (16, 4):
+        model(ids, model.new_cache(8, 40, spec_slots=slots))
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    assert set(grids) == {0, cus} and grids == sorted(grids, reverse=True)
+
+
 def test_mtp_forward_and_chain(micro):
     model, mtp, (W, W16), cfg = micro
     g = torch.Generator().manual_seed(3)

@@ -16,6 +16,7 @@ import functools
 
 import torch
 import torch.nn.functional as F
+from torch.autograd import forward_ad
 
 from .. import ops
 from .config import Qwen3_5Config
@@ -63,6 +64,19 @@ def gemm_grid(N, cus, rows=ops.GEMM_MAX_ROWS):
     return cus
 
 
+def opaque_call_ok(x, weight):
+    """Whether x W^T may be a call that PyTorch does not see: no gradient can reach x or the weight
+    (a trainable weight also changes, and its tiled copy does not), and no forward-mode level,
+    function transform, trace, compilation or dispatch mode is there to follow the operator."""
+    return (type(x) in (torch.Tensor, torch.nn.Parameter) and not weight.requires_grad
+            and not (x.requires_grad and torch.is_grad_enabled())
+            and forward_ad._current_level < 0
+            and torch._C._functorch.peek_interpreter_stack() is None
+            and torch._C._get_tracing_state() is None
+            and not torch._C._len_torch_dispatch_stack()
+            and not torch.compiler.is_compiling())
+
+
 class Projection:
     """y = x W^T (blocks.py's nn.Linear layers, no bias).  Keeps the row-major weight
     for hipBLASLt (F.linear) and a tiled copy for lollm_gemm (<= 64 rows) and
@@ -93,9 +107,9 @@ class Projection:
     def rows_plan(self, x, rows):
         """(tile, K parts) of lollm_gemm_rows for a call past the few-row GEMM, tile 0 for
         hipBLASLt: a pure function of the shape (and 0 where only F.linear serves: another
-        dtype, a gradient)."""
-        if (self.tiled is None or x.dtype != torch.bfloat16 or not x.is_cuda
-                or x.data_ptr() % 16 or (x.requires_grad and torch.is_grad_enabled())):
+        dtype, opaque_call_ok)."""
+        if (self.tiled is None or not opaque_call_ok(x, self.weight)
+                or x.dtype != torch.bfloat16 or not x.is_cuda or x.data_ptr() % 16):
             return 0, 1
         tile = ops.gemm_rows_tile(rows, self.N, self.K, self.epilogue, _cus())
         if tile:

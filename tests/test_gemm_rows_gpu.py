@@ -82,6 +82,69 @@ def test_projection_takes_the_rows_kernel_and_keeps_gradients():
 
 
 @pytest.mark.gpu
+def test_projection_keeps_weight_gradients_and_tangents():
+    """Past 64 rows a trainable weight gets its gradient and its updated values are used (also
+    without grad mode), and a forward-mode tangent passes: F.linear's, by exact equality."""
+    from torch.autograd import forward_ad
+    from lollm_amd.qwen3_5.blocks import Projection
+    print("case projection weight gradient and tangent", flush=True)
+    x, W = case(1200, 8192, 256, seed=6)
+    xd, Wd = x.cuda(), W.cuda()
+    wp = torch.nn.Parameter(Wd.clone())
+    p = Projection(wp)
+    p(xd).float().sum().backward()
+    want = torch.nn.Parameter(Wd.clone())
+    torch.nn.functional.linear(xd, want).float().sum().backward()
+    assert torch.equal(wp.grad, want.grad)
+    with torch.no_grad():
+        wp.mul_(2)
+        assert torch.equal(p(xd), torch.nn.functional.linear(xd, wp))
+    plain, dx = Projection(Wd), x.flip(0).cuda()
+    with forward_ad.dual_level():
+        tangent = forward_ad.unpack_dual(plain(forward_ad.make_dual(xd, dx))).tangent
+    assert torch.equal(tangent, torch.nn.functional.linear(dx, Wd))
+
+
+class _Recorded(torch.Tensor):
+    pass
+
+
+def test_opaque_call_rule():
+    """Each way in which PyTorch follows an operator keeps F.linear (on the CPU: the rule is
+    asked inside the transform, and the projection there equals F.linear's own result)."""
+    from torch.autograd import forward_ad
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from lollm_amd.qwen3_5.blocks import Projection, opaque_call_ok
+    x, W = case(70, 64, 128, seed=7)
+    p = Projection(W)
+    asked = []
+
+    def f(a):
+        asked.append(opaque_call_ok(a, W))
+        return p(a)
+
+    want = torch.nn.functional.linear(x, W)
+    assert torch.equal(f(x), want) and asked == [True]
+    with torch.inference_mode():
+        f(x)
+    with torch.no_grad():
+        f(x.clone().requires_grad_())
+    assert asked == [True] * 3
+    del asked[:]
+    assert not opaque_call_ok(x, torch.nn.Parameter(W))
+    assert f(x.clone().requires_grad_()).requires_grad
+    assert f(x.as_subclass(_Recorded)).shape == want.shape
+    batched = torch.func.vmap(f)(torch.stack([x, -x]))
+    torch.testing.assert_close(batched[1], -want)
+    assert torch.equal(torch.func.jvp(f, (x,), (x,))[1], want)
+    with forward_ad.dual_level():
+        assert torch.equal(forward_ad.unpack_dual(f(forward_ad.make_dual(x, x))).tangent, want)
+    assert torch.equal(make_fx(f)(x)(-x), torch.nn.functional.linear(-x, W))
+    assert torch.equal(torch.jit.trace(f, (x,), check_trace=False)(-x), torch.nn.functional.linear(-x, W))
+    assert asked == [False] * len(asked) and len(asked) >= 7
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K,splits,epi", [(65, 320, 1536, 12, 0), (129, 256, 512, 4, 0), (257, 1088, 384, 3, 0),
                                               (96, 4096, 8192, 16, 0), (100, 448, 256, 2, 1), (300, 8192, 256, 2, 0)])
 def test_gemm_rows_split_k(M, N, K, splits, epi):

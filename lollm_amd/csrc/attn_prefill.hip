@@ -74,12 +74,17 @@ __device__ __forceinline__ void ap_mfma(f32x16& s, bf16x8 k, bf16x8 q) {
 // the wait states between the last product and the first VALU access of its result
 __device__ __forceinline__ void ap_mfma_done(f32x16& s) { asm volatile("s_nop 15\n\ts_nop 7" : "+v"(s)); }
 
-// A pair of fp32 weights as bf16 hi and lo, x = hi + lo to 16 bits.
+// A pair of fp32 weights as bf16 hi and lo, x = hi + lo to 16 bits.  hi is cut and not rounded, so
+// that lo is never negative, and lo is at least 2^-126 where hi is not 0: an infinite V then takes
+// the sum of both products to infinity as a single product does, not to infinity - infinity or
+// 0 x infinity.
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ void ap_split(float x, float y, uint32_t& hi, uint32_t& lo) {
-  const bf16x2 h = {(__bf16)x, (__bf16)y};
-  hi = __builtin_bit_cast(uint32_t, h);
-  const bf16x2 l = {(__bf16)(x - __uint_as_float(hi << 16)), (__bf16)(y - __uint_as_float(hi & 0xffff0000u))};
-  lo = __builtin_bit_cast(uint32_t, l);
+  const uint32_t xb = __float_as_uint(x), yb = __float_as_uint(y);
+  hi = __builtin_amdgcn_perm(yb, xb, 0x07060302u);   // the upper halves
+  const bf16x2 l = {(__bf16)(x - __uint_as_float(xb & 0xffff0000u)), (__bf16)(y - __uint_as_float(yb & 0xffff0000u))};
+  const u16x2 least = __builtin_elementwise_min(__builtin_bit_cast(u16x2, hi), u16x2{0x0080, 0x0080});
+  lo = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, l), least));
 }
 __device__ __forceinline__ int ap_div(int r, uint32_t mul) { return (int)(((uint32_t)r * mul) >> 16); }
 

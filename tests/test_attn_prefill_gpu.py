@@ -78,7 +78,7 @@ def test_two_row_groups_match_oracle():
 @pytest.mark.parametrize("scale", [1.0, 2.0])
 def test_long_call_error_is_the_output_rounding(B, T, Hq, Hkv, L, scale):
     """Against 64 bits: the weights carry 16 bits and their sum 24, so the error is that of
-    rounding the exact result to bf16 (2^-17 of the weights beside it: under 1% of it); the
+    rounding the exact result to bf16 (2^-16 of the weights beside it: under 1% of it); the
     split kernels, whose weights carry 8 bits, are further away."""
     from lollm_amd import ops
     print(f"case long attention error B={B} T={T} L={L} scale={scale}", flush=True)
@@ -98,6 +98,27 @@ def test_long_call_error_is_the_output_rounding(B, T, Hq, Hkv, L, scale):
             err_split += (split[b, :, h] - o).square().sum().item()
             rounding += (o.bfloat16().double() - o).square().sum().item()
     assert err <= 1.02 * rounding and err <= err_split
+
+
+@pytest.mark.parametrize("B,T,Hq,Hkv", [(10, 100, 32, 4), (16, 231, 32, 4)])
+def test_infinite_values_stay_infinite(B, T, Hq, Hkv):
+    """Infinite and NaN V entries reach the rows that see them as they are (key 0: every row, the
+    first with a weight of exactly 1), as from the split kernels, and no other column."""
+    from lollm_amd import ops
+    print(f"case infinite values B={B} T={T}", flush=True)
+    q, kc, vc, kl, gate = make_case(B, T, Hq, Hkv, [T] * B, seed=B + T)
+    clean = long_call(q, kc, vc, kl, gate)
+    inf, nan, late = float("inf"), float("nan"), 37
+    vc[:, :, 0, 3], vc[:, :, 0, 200], vc[:, :, 0, 64] = inf, -inf, nan
+    vc[:, :, late, 5], vc[:, :, late, 130] = -inf, inf
+    out = long_call(q, kc, vc, kl, gate)
+    split = ops.attn_verify(q.cuda(), kc.cuda(), vc.cuda(), kl.cuda(), gate.cuda(), grid=256)
+    out, split, clean = (t.cpu().float().view(B, T, Hq, D) for t in (out, split, clean))
+    for o in (out, split):
+        assert (o[..., 3] == inf).all() and (o[..., 200] == -inf).all() and o[..., 64].isnan().all()
+        assert (o[:, late:, :, 5] == -inf).all() and (o[:, late:, :, 130] == inf).all()
+    rest = [c for c in range(D) if c not in (3, 200, 64, 5, 130)]
+    assert torch.equal(out[..., rest], clean[..., rest])
 
 
 def test_large_scores_move_the_reference_maximum():

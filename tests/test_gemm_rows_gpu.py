@@ -146,11 +146,14 @@ def test_opaque_call_rule():
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K,splits,epi", [(65, 320, 1536, 12, 0), (129, 256, 512, 4, 0), (257, 1088, 384, 3, 0),
-                                              (96, 4096, 8192, 16, 0), (100, 448, 256, 2, 1), (300, 8192, 256, 2, 0)])
+                                              (96, 4096, 8192, 16, 0), (100, 448, 256, 2, 1), (300, 8192, 256, 2, 0),
+                                              (300, 8192, 512, 4, 0)])
 def test_gemm_rows_split_k(M, N, K, splits, epi):
     """K in parts: each part's fp32 sums added in order, one rounding at the end.  The last case
-    has more (tile, part) pairs than CUs."""
+    has more (tile, part) pairs than CUs, so that workgroups go from one to the next."""
     from lollm_amd import ops
+    if splits == 4 and M == 300:
+        assert -(-M // 128) * -(-N // 256) * splits > torch.cuda.get_device_properties(0).multi_processor_count
     print(f"case gemm rows split M={M} N={N} K={K} splits={splits} epi={epi}", flush=True)
     x, W = case(M, N, K, seed=M + K)
     W, xd = (W.float() * 3).bfloat16().cuda(), x.cuda()

@@ -49,20 +49,16 @@ class MTP:
                                [self.fc] + layer.self_attn.projections() + layer.mlp.projections()),
                            model.device)
 
-    def _block(self, hidden, next_emb, k_cache, v_cache, lengths, kv_len, rope_pos, ws, tok=None,
+    def _block(self, hidden, k_cache, v_cache, lengths, kv_len, rope_pos, ws, tok=None,
                fc_in=None):
-        """Returns (MTP layer output before the final norm, normed output).  Given the
-        next tokens' ids `tok` (B,) int32 instead of their embeddings, the lookup, both
-        pre-fc norms and the concatenation run as one kernel (lollm_mtp_input); fc_in: that
-        input, formed already."""
-        if fc_in is None and tok is not None:
+        """Returns (MTP layer output before the final norm, normed output).  The fc input is
+        `fc_in`, or from the next tokens' ids `tok` (B,) int32: the lookup, both pre-fc norms
+        and the concatenation run as one kernel (lollm_mtp_input)."""
+        if fc_in is None:
             B = tok.numel()
             fc_in = ops.mtp_input(tok, hidden, self.model.model.embed_tokens.weight,
                                   self.pre_fc_norm_embedding.weight, self.pre_fc_norm_hidden.weight,
                                   self.pre_fc_norm_embedding.eps).view(B, 1, -1)
-        elif fc_in is None:
-            fc_in = torch.cat([self.pre_fc_norm_embedding(next_emb),
-                               self.pre_fc_norm_hidden(hidden)], -1)
         layer = self.layers[0]
         # fc and the layer's input_layernorm (the fc output starts the residual stream)
         h_in, x = self.fc.add_norm(fc_in, None, layer.input_layernorm)
@@ -101,7 +97,7 @@ class MTP:
         shape = (B, self.cfg.num_key_value_heads, L, self.cfg.head_dim)
         kc = torch.empty(shape, dtype=torch.bfloat16, device=dev)
         vc = torch.empty(shape, dtype=torch.bfloat16, device=dev)
-        _, normed = self._block(hidden, next_emb, kc, vc, zeros, kv_len, rope, None, fc_in=fc_in)
+        _, normed = self._block(hidden, kc, vc, zeros, kv_len, rope, None, fc_in=fc_in)
         return normed
 
     __call__ = forward
@@ -245,7 +241,7 @@ class SpecDecoder:
         tok = self.pending
         h = self.h_last.view(B, 1, -1)
         for j in range(1, k + 1):
-            m, normed = mtp._block(h, None, self.mkc, self.mvc, self.mtp_len[j - 1],
+            m, normed = mtp._block(h, self.mkc, self.mvc, self.mtp_len[j - 1],
                                    self.mtp_len[j], self.mtp_len[j], self.mtp_ws, tok=tok)
             lm = model.lm_head
             if self.draft_mode == "sample":

@@ -83,16 +83,21 @@ class Qwen3_5Model:
     def new_cache(self, batch, max_len, spec_slots=4):
         return Qwen3_5Cache(self.cfg, batch, max_len, spec_slots, self.device)
 
-    def attn_workspace(self, B, T, max_len):
+    def attn_workspace(self, B, T, max_len, keep=True):
         """Split-K partials buffer of the attention layers (shared by all layers of a
-        call; one per (B, T) shape, kept for graph replays)."""
+        call; one per (B, T) shape, kept for graph replays).  keep=False: the caller's own,
+        for the prompts, of which there are as many shapes as lengths (16 x 2048 tokens,
+        4 KV heads of 8 query heads: 1.1 GB)."""
         cfg = self.cfg
         key = (B, T, max_len, self.attn_grid)
-        if key not in self._ws:
+        ws = self._ws.get(key)
+        if ws is None:
             n = ops.attn_workspace_bytes(B, T, cfg.num_attention_heads, cfg.num_key_value_heads,
                                          cfg.head_dim, max_len, self.attn_grid)
-            self._ws[key] = torch.empty(max(n, 16), dtype=torch.uint8, device=self.device)
-        return self._ws[key]
+            ws = torch.empty(max(n, 16), dtype=torch.uint8, device=self.device)
+            if keep:
+                self._ws[key] = ws
+        return ws
 
     @torch.no_grad()
     def forward(self, input_ids, past=None, return_hidden=False, logits="all"):
@@ -124,7 +129,8 @@ class Qwen3_5Model:
             h_first = None
         else:
             x, h_first, kv_len = inputs
-        ws = self.attn_workspace(B, T, cache.max_len)
+        # (the calls that repeat a shape: one token, the verify block)
+        ws = self.attn_workspace(B, T, cache.max_len, keep=T <= max(cache.spec_slots, 1))
         # a call that can be rolled back (the verify block, as the GDN layers tell it) asks for
         # the split-K attention at any size, where a row's bits do not depend on T
         grid = self.attn_grid or (_cus() if T <= cache.spec_slots else 0)

@@ -130,6 +130,21 @@ def test_verify_block_asks_for_the_split_attention(micro, monkeypatch):
     assert set(grids) == {0, cus} and grids == sorted(grids, reverse=True)
 
 
+def test_prompts_leave_no_attention_workspace_behind(micro):
+    """The model keeps the attention workspace of the calls that repeat their shape (one token,
+    the verify block), not one for every prompt length it meets."""
+    model, _, _, cfg = micro
+    print("case prompt workspaces", flush=True)
+    cache = model.new_cache(1, 200)
+    step = torch.zeros(1, 1, dtype=torch.long, device="cuda")
+    model(step, cache)
+    kept = dict(model._ws)
+    for n in (5, 17, 40, 70):
+        model(torch.zeros(1, n, dtype=torch.long, device="cuda"), cache)
+    model(step, cache)
+    assert set(model._ws) == set(kept) and all(model._ws[k] is kept[k] for k in kept)
+
+
 def test_mtp_forward_and_chain(micro):
     model, mtp, (W, W16), cfg = micro
     g = torch.Generator().manual_seed(3)

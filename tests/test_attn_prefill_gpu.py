@@ -132,6 +132,31 @@ def test_large_scores_move_the_reference_maximum():
     torch.testing.assert_close(out.cpu().float(), oracle(q, kc, vc, kl, gate), **TOL)
 
 
+@pytest.mark.parametrize("B,T,Hq,Hkv", [(10, 100, 10, 2), (16, 231, 32, 4)])
+def test_cache_strides_beyond_packed(B, T, Hq, Hkv):
+    """Heads and sequences of the caches further apart than packed (the library's strides; NaN in
+    the gaps), in both tile heights: the bits of the packed caches."""
+    from lollm_amd import _lib, ops
+    print(f"case long attention strides B={B} T={T}", flush=True)
+    q, kc, vc, kl, gate = make_case(B, T, Hq, Hkv, [T + 2 * b for b in range(B)], seed=T)
+    packed = long_call(q, kc, vc, kl, gate)
+    n = kc.shape[2]
+    head, seq = (n + 3) * D, Hkv * (n + 3) * D + 5 * D
+    wide = []
+    for c in (kc, vc):
+        buf = torch.full((B * seq,), float("nan"), dtype=torch.bfloat16, device="cuda")
+        buf.as_strided((B, Hkv, n, D), (seq, head, D, 1)).copy_(c)
+        wide.append(buf)
+    qd, gd, kld, out = q.cuda(), gate.cuda(), kl.cuda(), torch.zeros_like(packed)
+    need = ops.attn_workspace_bytes(B, T, Hq, Hkv, D, n)
+    ws = torch.full((need,), 0x5A, dtype=torch.uint8, device="cuda")
+    p = ops._ptr
+    rc = _lib.lib().lollm_attn_verify(p(qd), p(wide[0]), p(wide[1]), p(kld), p(gd), p(out), p(ws), need, B, T, Hq,
+                                      Hkv, D, n, seq, head, 0, D ** -0.5, ops._stream())
+    assert rc == 0
+    assert torch.equal(out, packed) and bool((ws == 0x5A).all())
+
+
 @pytest.mark.parametrize("B,T,Hq,Hkv,rd,rope", [(2, 150, 8, 2, 64, None), (4, 64, 5, 2, 256, "start"),
                                                (3, 100, 4, 1, 16, "token"), (2, 128, 3, 3, 0, None),
                                                (2, 130, 4, 2, 128, "token")])

@@ -11,12 +11,22 @@ D, K = 128, 4
 
 
 def call(ops, m, spread, fresh, monkeypatch):
+    """One long call in the spread or the walked form (also where the rule would take the other),
+    held to that kernel's entry."""
+    from lollm_amd import _lib
     monkeypatch.setattr(ops, "GDN_SPLIT_MAX_HEADS", 1 << 30 if spread else 0)
+    monkeypatch.setattr(ops, "GDN_CHUNK", 0)
+    ran = []
+    for name in ("lollm_gdn_layer_split", "lollm_gdn_layer_chunked"):
+        fn = getattr(_lib.lib(), name)
+        monkeypatch.setattr(_lib.lib(), name, lambda *a, fn=fn, name=name: ran.append(name) or fn(*a))
     win, rec = m["win"].clone(), m["rec"].clone()
     out = ops.gdn_layer(m["proj"], m["conv_w"], m["A_log"], m["dt_bias"], m["norm_w"], win, m["off"], rec,
                         m["half"], m["rep"], m["replay"], fresh, m["B"], m["T"], m["Hk"], m["Hv"], D, K, 1e-6,
                         chunked=True)
     torch.cuda.synchronize()
+    monkeypatch.undo()
+    assert ran == ["lollm_gdn_layer_split" if spread else "lollm_gdn_layer_chunked"]
     return out.float().cpu(), rec.cpu(), win.cpu()
 
 
